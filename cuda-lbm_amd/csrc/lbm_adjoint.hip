@@ -205,10 +205,12 @@ int lbm_adjoint_forward(lbm_ctx* ctx, int32_t nsteps, int32_t every) {
                                           ctx->stream);
             if (e != hipSuccess) return ctx->hip_fail(e, "checkpoint copy");
         }
-        // a pair of steps per launch unless a checkpoint falls between them
-        if (pairs && t + 2 <= nsteps && (t + 1) % every != 0) {
-            rc = ctx->two_step(t + 2 == nsteps);
-            t += 2;
+        // several steps per launch up to the next checkpoint
+        const int left = every - t % every < nsteps - t ? every - t % every : nsteps - t;
+        if (pairs && left >= 2) {
+            int n = 0;
+            rc = ctx->multi_step(left, t + left == nsteps, &n);
+            t += n;
         } else {
             rc = ctx->one_step(t == nsteps - 1);
             t += 1;

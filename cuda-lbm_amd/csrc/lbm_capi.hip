@@ -223,9 +223,10 @@ bool lbm_ctx::two_step_ok() const {
     return cfg.steps_per_launch != 1 && !adapt && !ibm.active && !(cfg.quirks & LBM_QUIRK_STALE_REST) && flags_local;
 }
 
-// Two steps from buf[cur] into buf[1-cur] in one launch (the same arithmetic as two
-// one-step launches).
-int lbm_ctx::two_step(bool write_macros) {
+// Two or more steps from buf[cur] into buf[1-cur] in one launch (the same arithmetic as as
+// many one-step launches): at most steps_left >= 2, *done of them. `last`: the run ends with
+// the steps_left steps, so a launch that takes them all stores the fields.
+int lbm_ctx::multi_step(int steps_left, bool last, int* done) {
     hipError_t e;
     ahead_valid = ahead_edges = false;
     if (n_edge > 0 && !edge_in_store) {  // state t-1 at the edge nodes: buf[1-cur] -> store
@@ -233,19 +234,26 @@ int lbm_ctx::two_step(bool write_macros) {
                              cfg.periodic_y, 1, stream);
         if (e != hipSuccess) return hip_fail(e, "edge save launch");
     }
+    MarchPolicy mp;
+    if (flags_march) mp = march_policy(cfg.nx, cfg.ny, plane, cfg.storage, cfg.collision, d_flags || n_edge > 0, steps_left);
+    const int n = mp.steps ? mp.steps : 2;
+    const bool write_macros = last && n == steps_left;
     StepParams p = step_params(cur, write_macros);
     p.edge_prev = d_edge[edge_cur];
     p.edge_next = d_edge[1 - edge_cur];
     p.n_edge = n_edge;
-    e = launch_step2(cfg.collision, cfg.storage, p, step2_policy(plane, cfg.storage, cfg.collision), stream);
-    if (e != hipSuccess) return hip_fail(e, "two-step launch");
+    p.edge_all = steps_left - n < 2;  // else the next launch of this call saves them
+    if (mp.steps) e = launch_march(cfg.collision, cfg.storage, p, mp, d_row_info, stream);
+    else e = launch_step2(cfg.collision, cfg.storage, p, step2_policy(plane, cfg.storage, cfg.collision), stream);
+    if (e != hipSuccess) return hip_fail(e, "multi-step launch");
     if (n_edge > 0) {
         edge_cur = 1 - edge_cur;
         edge_in_store = true;
     }
     cur = 1 - cur;
-    timestep += 2;
+    timestep += n;
     if (write_macros) macros_valid = true;
+    *done = n;
     return LBM_OK;
 }
 
@@ -525,8 +533,8 @@ int lbm_set_flags(lbm_ctx* ctx, const uint8_t* flags, int on_device) {
     } else {
         std::memcpy(h.data(), flags, ctx->N);
     }
-    std::vector<uint8_t> rowc(size_t(ny), 0);
-    bool any = false, local = true;
+    std::vector<uint8_t> rowc(size_t(ny) * 2, 0);  // row classes, then march_row_info()
+    bool any = false, local = true, march = true;
     for (int y = 0; y < ny; y++) {
         for (int x = 0; x < nx; x++) {
             uint8_t f = h[size_t(y) * nx + x];
@@ -535,6 +543,7 @@ int lbm_set_flags(lbm_ctx* ctx, const uint8_t* flags, int on_device) {
             if (f == LBM_FLUID) continue;
             any = true;
             if (flag_reads_neighbour(f)) local = false;
+            if (!march_flag(f)) march = false;
             if (f == LBM_PRESSURE_OUTLET) {
                 // reads the post-stream populations of (x - 1, y); as for ZG_OUTFLOW, none of
                 // them may be an unstreamed slot (another thread writes that slot)
@@ -578,18 +587,21 @@ int lbm_set_flags(lbm_ctx* ctx, const uint8_t* flags, int on_device) {
         (void)hipFree(ctx->d_flags);
         (void)hipFree(ctx->d_row_class);
         ctx->d_flags = nullptr;
-        ctx->d_row_class = nullptr;
+        ctx->d_row_class = ctx->d_row_info = nullptr;
     }
     ctx->flags_local = local;
+    ctx->flags_march = march;
     if (!any) return LBM_OK;
     row_classes(h.data(), nx, ny, rowc.data());
+    march_row_info(h.data(), rowc.data(), nx, ny, rowc.data() + ny);
     rc = ctx->dev_alloc(reinterpret_cast<void**>(&ctx->d_flags), ctx->N, "flags");
     if (rc) return rc;
-    rc = ctx->dev_alloc(reinterpret_cast<void**>(&ctx->d_row_class), size_t(ny), "row classes");
+    rc = ctx->dev_alloc(reinterpret_cast<void**>(&ctx->d_row_class), size_t(ny) * 2, "row classes");
     if (rc) return rc;
+    ctx->d_row_info = ctx->d_row_class + ny;
     rc = ctx->upload(ctx->d_flags, h.data(), ctx->N, 0);
     if (rc) return rc;
-    return ctx->upload(ctx->d_row_class, rowc.data(), size_t(ny), 0);
+    return ctx->upload(ctx->d_row_class, rowc.data(), size_t(ny) * 2, 0);
 }
 
 int lbm_init_from_macros(lbm_ctx* ctx, const float* rho, const float* u, int on_device) {
@@ -662,8 +674,8 @@ int lbm_step(lbm_ctx* ctx, int32_t nsteps) {
     if (rc) return rc;
     int i = 0;
     if (ctx->two_step_ok())
-        for (; i + 2 <= nsteps; i += 2) {
-            rc = ctx->two_step(i + 2 == nsteps);
+        for (int n = 0; i + 2 <= nsteps; i += n) {
+            rc = ctx->multi_step(nsteps - i, true, &n);
             if (rc) return rc;
         }
     for (; i < nsteps; i++) {

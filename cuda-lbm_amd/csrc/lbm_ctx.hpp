@@ -95,8 +95,10 @@ struct lbm_ctx {
     int edge_cur = 0;
     bool edge_in_store = false;
     bool flags_local = true;           // no flag needs a neighbour's populations
+    bool flags_march = true;           // every flag's functor is one a marching launch applies
     uint8_t* d_flags = nullptr;
     uint8_t* d_row_class = nullptr;
+    uint8_t* d_row_info = nullptr;     // march_row_info(), in d_row_class's allocation
     float* d_force_field = nullptr;
     float *d_rho = nullptr, *d_ux = nullptr, *d_uy = nullptr;
     float* d_avg = nullptr;
@@ -137,7 +139,7 @@ struct lbm_ctx {
     int ibm_graph_pair();
     void ibm_graph_free();
     bool two_step_ok() const;
-    int two_step(bool write_macros);
+    int multi_step(int steps_left, bool last, int* done);
     int restore_edges();
     // lbm_ibm.hip
     int ibm_pass(int src_idx);

@@ -2,6 +2,7 @@
 #include "lbm_kernels.hpp"
 
 #include <hip/hip_runtime.h>
+#include <cmath>
 
 namespace lbm {
 
@@ -566,6 +567,77 @@ Step2Policy step2_policy(long long plane, int storage, int coll) {
         }
     }
     return lp;
+}
+
+// Measured on MI355X, us per step, 48-step calls, against the two-step forms (tiles or strips)
+// of the same build and box; S x w x h the marching shape:
+//   periodic   64^2 BGK F32  2.41 -> 1.58 (4x58x1)     128^2 2.33 -> 1.71 (4x58x1)
+//   periodic  512^2 BGK F32  4.11 -> 3.00 (4x58x3)     1024^2 MRT F32 9.52 -> 6.51 (4x58x10)
+//   periodic  4096x1024 BGK F32 35.3 -> 15.4 (6x54)    3000x2500 CM F32 87.3 -> 40.6 (4x58)
+//   periodic 8192^2 F32: BGK 505 -> 223 (6x48x32 wide; 6x54x32 259, 4x48x32 312),
+//                        MRT 511 -> 256..262 (6x48x48, 6x54x32), CM 530 -> 308 (6x54x32; 4x48x32 336)
+//   periodic 8192^2 F16: BGK 336 -> 215..220 (4x58), MRT 361 -> 245
+//   channel   4096x1024 CM BF16 36.7 -> 28 (4x58), MRT F32 41.8 -> 24 (4x58x24; 6x54x16 25.5)
+//   cavity    1024^2 MRT F32 11.1 -> 9.3 (4x58x10)     4000x3000 BGK F32 107 -> 49 (6x54x32; 4x58x32 64)
+//   cavity    2048^2 MRT F16 36.0 -> 25.3, F32 45.1 -> 24.1 (4x58)
+//   walls on small grids: cavity 512^2 5.08 -> 5.14, 256^2 CM 3.55 -> 4.31, 6000x60 5.50 -> 5.93,
+//   channel 700^2 CM 6.43 -> 7.31, cavity 777x611 MRT F16 6.6 -> 7.0: there the strips along the
+//   walls are a large share and set the launch time, so up to 48 MB walled grids keep the tiles.
+// Six steps pay once the populations leave the Infinity Cache (the launch is then bound by HBM
+// at four steps, by the vector ALU at six), later for CM (more arithmetic) and walled grids.
+// Aligned 48-column strips, four to a workgroup, write whole 64-byte granules and keep the
+// neighbours' shared lines in L2; the 14 % of lanes they idle only pay in HBM and for BGK.
+// The height balances the halo rows (S - 1 + h per h) against the number of wavefronts: the cost
+// is wavefronts per SIMD, rounded up, times rows, with a penalty for one or two wavefronts per
+// SIMD, which leave the vector ALU idle while they wait.
+MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll, bool edge, int steps_left) {
+    MarchPolicy lp;
+    const bool f32 = storage == LBM_F32;
+    if (nx < kMarchMinSide || ny < kMarchMinSide || steps_left < 4) return lp;
+    // populations are addressed through one buffer resource
+    if (!(f32 ? buf_fits<float>(Q, plane) : buf_fits<uint16_t>(Q, plane))) return lp;
+    const double bytes = 2.0 * 9.0 * double(plane) * (f32 ? 4.0 : 2.0);
+    if (edge && bytes <= 48.0e6) return lp;
+    const bool six = f32 && steps_left >= 6 && bytes > (edge || coll == LBM_CM ? 600.0e6 : 256.0e6);
+    lp.steps = six ? 6 : 4;
+    lp.w = kMarchLanes - 2 * (lp.steps - 1);
+    if (bytes > 600.0e6) {
+        lp.h = 32;
+        if (six && coll == LBM_BGK && nx % 16 == 0) {
+            lp.w = 48;
+            lp.wide = true;
+        }
+        return lp;
+    }
+    const long long sx = (nx + lp.w - 1) / lp.w;
+    const int resident = edge ? 4 : 5;  // wavefronts per SIMD
+    double best = 1e30;
+    for (int h = 1; h <= 48; h++) {
+        const double n = double(sx * ((ny + h - 1) / h)) / double(kSimds), rows = h + lp.steps - 1;
+        const double c = std::ceil(n);
+        const double idle = c <= 1 ? 1.7 : (c <= 2 ? 1.1 : (c <= 3 ? 1.03 : 1.0));
+        const double cost = (c <= resident ? c * idle : n + 0.5) * rows;
+        if (cost < best) {
+            best = cost;
+            lp.h = h;
+        }
+    }
+    return lp;
+}
+
+hipError_t launch_march(int coll, int storage, const StepParams& p, const MarchPolicy& lp, const uint8_t* row_info, hipStream_t s) {
+    if (p.n_edge != edge_count(p.nx, p.ny, p.px, p.py)) return hipErrorInvalidValue;
+    if (p.n_edge > 0 && (!p.edge_prev || !p.edge_next)) return hipErrorInvalidValue;
+    if (p.nx < kMarchMinSide || p.ny < kMarchMinSide || lp.w < 1 || lp.w > kMarchLanes - 2 * (lp.steps - 1) || lp.h < 1 ||
+        lp.h + 2 * (lp.steps - 1) > kMarchMaxRows)
+        return hipErrorInvalidValue;
+    const long long sx = (p.nx + lp.w - 1) / lp.w, n = sx * ((p.ny + lp.h - 1) / lp.h);
+    if (n > 0x7fffff00LL) return hipErrorInvalidValue;
+    const MarchGrid m{int(sx), int(n), lp.w, lp.h, row_info, 0};
+    const bool edge = p.flags || !p.px || !p.py;
+    if (storage == LBM_F16_SHIFTED) return launch_march_f16(coll, lp.steps, p, m, edge, lp.wide, s);
+    if (storage == LBM_BF16_SHIFTED) return launch_march_bf16(coll, lp.steps, p, m, edge, lp.wide, s);
+    return launch_march_f32(coll, lp.steps, p, m, edge, lp.wide, s);
 }
 
 hipError_t launch_edge_copy(int storage, void* buf, void* store, long long plane, int nx, int ny, int px, int py,

@@ -3,11 +3,12 @@
 
 #include <hip/hip_runtime.h>
 
-#include "lbm_step.hpp"
+#include "lbm_march.hpp"
 
 namespace lbm {
 
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, workgroups dealt round-robin
+constexpr int kSimds = 1024;  // 256 compute units of four SIMDs
 
 struct InitParams {
     const float* rho;  // [N]
@@ -46,6 +47,19 @@ struct Step2Policy {
 Step2Policy step2_policy(long long plane, int storage, int coll);
 long long step2_grid_blocks(const StepParams& p, const Step2Policy& lp);
 hipError_t launch_step2(int coll, int storage, const StepParams& p, const Step2Policy& lp, hipStream_t s);
+// Several steps per launch in marching strips (lbm_march.hpp). steps 0: not for this grid (the
+// two-step forms run). p as for launch_step2; p.mid, when set, receives the steps - 1
+// intermediate states, mid_stride elements apart.
+struct MarchPolicy {
+    int steps = 0;
+    int w = 0, h = 0;  // columns and rows per strip
+    bool wide = false; // four strips per workgroup instead of one
+};
+MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll, bool edge, int steps_left);
+hipError_t launch_march(int coll, int storage, const StepParams& p, const MarchPolicy& lp, const uint8_t* row_info, hipStream_t s);
+hipError_t launch_march_f32(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s);
+hipError_t launch_march_f16(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s);
+hipError_t launch_march_bf16(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s);
 // to_store = 1: edge nodes of `buf` -> store; 0: store -> edge nodes of `buf`.
 hipError_t launch_edge_copy(int storage, void* buf, void* store, long long plane, int nx, int ny, int px, int py,
                             int to_store, hipStream_t s);

@@ -1,0 +1,520 @@
+// lbm_march.hpp — several time steps per launch with the whole state in registers.
+//
+// One wavefront owns a strip of `w` columns x `h` rows, lane l = column x0 - (S-1) + l, and
+// marches up it one row per iteration, on its own: no LDS tile, no barrier. Iteration i runs S
+// stages: stage k advances row first + i - k (first = y0 - (S-1)) from state t+k to state
+// t+k+1. Stage 0 pulls from the source buffer (loaded one iteration ahead), stage k from the
+// rows stage k-1 has just produced: of the nine directions the three with c_y = -1 come from
+// the row of this iteration, the three with c_y = 0 from the row before, the three with
+// c_y = +1 from the one before that, so a stage keeps nine values per lane, and the x shift is
+// one cross-lane move per direction with c_x != 0. The last stage stores state t+S. A
+// population crosses HBM once per S steps; the price is 2 (S-1) lanes and 2 (S-1-k) extra rows
+// per strip in stage k.
+//
+// Unstreamed slots (a source outside a non-periodic domain: the slot keeps the state two steps
+// older, see lbm_step.hpp): stage 0 reads state t-1 from the edge store, stage 1 reads state t
+// from the source buffer, stage k >= 2 the output of stage k-2 at its own node, which edge
+// lanes and edge rows leave in a small array of the wavefront (MarchHist). The launch saves
+// state t+S-1 of its own edge nodes for the next launch's stage 0.
+//
+// What bounds it: the vector ALU on grids of two or more wavefronts per SIMD, and below that
+// the wavefront's own instruction stream, scalar instructions included (a wavefront issues one
+// instruction per four cycles whatever its kind). Hence buffer addressing (one scalar add per
+// access), row offsets carried from row to row, and one bit mask that sends the rows needing
+// anything special (edges, walls, flags) out of the common path.
+//
+// The lane body is __host__ __device__; the GPU kernels (lbm_march_kernels.hpp) hold one lane
+// per thread, the host emulation 64 lanes in lockstep.
+#pragma once
+
+#include "lbm_step.hpp"
+
+#include <type_traits>
+
+namespace lbm {
+
+constexpr int kMarchLanes = 64;
+constexpr int kMarchMaxRows = 64;  // rows a strip touches: one bit each of the row masks
+constexpr int kMarchMinSide = 16;  // shorter grids would wrap more than once
+// Collision ids of the marching kernels: the operators, and MRT with the conserved moments'
+// rates zero (as every MRT scenario sets them; collide_mrt_t<true>).
+constexpr int kMarchMrtCons = 3;
+
+// Geometry of a launch (uniform).
+struct MarchGrid {
+    int strips_x, n_strips;
+    int w, h;                 // output columns and rows per strip
+    const uint8_t* row_info;  // march_row_info() of the flags, or null (all FLUID)
+    long long mid_stride;     // elements between the intermediate states at StepParams::mid
+};
+
+// What later stages read of earlier ones at unstreamed slots, per wavefront: for each stage
+// k <= S-3, the y group of rows 0 and NY-1 (all lanes) and a ring of three rows of the x group
+// of the lanes at x = 0 and NX-1.
+template <int S>
+struct MarchHist {
+    static constexpr int K = S > 2 ? S - 2 : 1;
+    float y[K][2][3][kMarchLanes];
+    float x[K][3][2][3];
+};
+
+// The x group and y group directions: those pulled from outside across the face (side 0: x = 0
+// or y = 0).
+LBM_HD constexpr int march_xq(int side, int j) { return side == 0 ? (j == 0 ? 1 : (j == 1 ? 5 : 8)) : (j == 0 ? 3 : (j == 1 ? 6 : 7)); }
+LBM_HD constexpr int march_yq(int side, int j) { return side == 0 ? (j == 0 ? 2 : (j == 1 ? 5 : 6)) : (j == 0 ? 4 : (j == 1 ? 7 : 8)); }
+
+// Flags whose functors a marching launch applies; grids with any other flag take the two-step
+// or one-step forms (the regularized functors rebuild the node from nine equilibria, which
+// every wavefront of the launch would pay for in registers).
+LBM_HD bool march_flag(uint8_t f) {
+    return f == LBM_FLUID || f == LBM_BOUNCE_BACK || f == LBM_MOVING_WALL_BOUNCE_BACK || f == LBM_ZOU_HE_TOP ||
+           f == LBM_ZOU_HE_LEFT || f == LBM_CYLINDER;
+}
+
+// Per row: bits 0-1 its row class (row_classes() in `classes`), 4 the node x = 0 is BOUNCE_BACK,
+// 8 the node x = NX-1 is; of rows 0 and NY-1 also 16 every node between them is BOUNCE_BACK, 32
+// every node between them is a moving wall.
+inline void march_row_info(const uint8_t* flags, const uint8_t* classes, int nx, int ny, uint8_t* out) {
+    for (int y = 0; y < ny; y++) {
+        const uint8_t* f = flags + (long long)y * nx;
+        int v = classes[y] | (f[0] == LBM_BOUNCE_BACK ? 4 : 0) | (f[nx - 1] == LBM_BOUNCE_BACK ? 8 : 0);
+        if (y == 0 || y == ny - 1) {
+            bool bb = true, mv = true;
+            for (int x = 1; x < nx - 1; x++) {
+                bb = bb && f[x] == LBM_BOUNCE_BACK;
+                mv = mv && f[x] == LBM_MOVING_WALL_BOUNCE_BACK;
+            }
+            v |= (bb ? 16 : 0) | (mv ? 32 : 0);
+        }
+        out[y] = uint8_t(v);
+    }
+}
+
+// The arguments as the special rows' code sees them: opaque there, so that nothing derived from
+// them (plane and slot offsets, array resources) is computed ahead and held across the march,
+// where it overflows the scalar registers into vector lanes (190 lane moves in the edge body).
+LBM_HD StepParams march_cold(const StepParams& p) {
+    StepParams c = p;
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(c.plane), "+s"(c.nx), "+s"(c.ny), "+s"(c.n_edge), "+s"(c.px), "+s"(c.py), "+s"(c.src));
+    asm volatile("" : "+s"(c.edge_prev), "+s"(c.edge_next), "+s"(c.flags), "+s"(c.quirks), "+s"(c.rho0));
+    asm volatile("" : "+s"(c.wall_ux), "+s"(c.wall_uy), "+s"(c.u_lid));
+#endif
+    return c;
+}
+
+// Masks over the rows a strip touches (bit i: row first + i), from look() of the 64 lanes.
+struct MarchRows {
+    uint64_t special;   // anything but plain fluid away from every edge
+    uint64_t straight;  // a straight wall: the x-edge nodes of a strip with an x edge, or the whole
+                        // row 0 or NY-1 of a strip without one; the rest of the row is fluid
+    uint64_t moving;    // ... row 0 or NY-1, moving
+    uint64_t flag;      // the flags of every node are read and their functors applied
+};
+
+// Lane state and the per-lane parts of an iteration. EDGE: the grid has a non-periodic axis or
+// boundary flags. FORCED: 0 no force, 1 the uniform force, 2 the force field. MODE 0: S steps;
+// MODE 1 (S = 2): one step and the next step's moment sums (CM<OptimalAdapter>): stage 0 stores
+// the step and its fields, stage 1 only sums; MODE 2: S steps, and StepParams::mid receives
+// the intermediate states.
+template <int COLL, int STORE, int S, bool EDGE, int FORCED, int MODE>
+struct MarchLane {
+    using St = Elem<STORE>;
+    using T = typename St::T;
+    static constexpr uint32_t B = sizeof(T);
+    using Buf = PopBuf<T, true>;
+
+    float g[Q];       // the stage at work: pulled populations in, post-collision out
+    float gn[Q];      // next row's stage-0 pulls
+    float up2[S][3], up1[S][3], mid1[S][3];  // delayed rows between stages (x-shifted already)
+    float fx[S], fy[S], fxn, fyn;            // FORCED 2: the force of each stage's row
+    float sx[2][3], sxn[2][3];               // EDGE: unstreamed x group of stages 0 and 1
+    std::conditional_t<(S > 4), uint64_t, uint32_t> fl;  // EDGE: flags of the last S rows, newest lowest
+    uint32_t fln;
+    uint32_t oc, om, op;                     // the lane's column and its x neighbours
+    int kind;                                // bits: 1 output column, 2 outside the domain, 4 x = 0, 8 x = NX-1 (unwrapped)
+    // uniform
+    int x0, y0, hs, first;
+    uint32_t om1, o0, op1;                   // element offsets of the rows below, at and above the next row to load
+    uint32_t od;                             // ... and of the row the last stage stores
+    int xany;                                // the strip holds an unwrapped x edge
+    MarchRows rows;
+
+    LBM_HD bool own() const { return (kind & 1) != 0; }
+    LBM_HD bool dead() const { return EDGE && (kind & 2) != 0; }
+    LBM_HD bool exl() const { return EDGE && (kind & 4) != 0; }
+    LBM_HD bool exr() const { return EDGE && (kind & 8) != 0; }
+    LBM_HD int iterations() const { return hs + 2 * (S - 1); }
+    LBM_HD bool row_in(const StepParams& p, int r) const { return !EDGE || p.py || (r >= 0 && r < p.ny); }
+    LBM_HD static bool bit(uint64_t m, int i) { return ((m >> i) & 1u) != 0; }
+
+    // Row r (at most one period off) in the grid; outside a non-periodic domain some row inside.
+    LBM_HD static int row_at(const StepParams& p, int r) {
+        if (EDGE && !p.py) return r < 0 ? 0 : (r >= p.ny ? p.ny - 1 : r);
+        return r < 0 ? r + p.ny : (r >= p.ny ? r - p.ny : r);
+    }
+    LBM_HD static uint32_t row_off(const StepParams& p, int r) { return uint32_t(row_at(p, r)) * uint32_t(p.nx); }
+
+    LBM_HD void init(const StepParams& p, const MarchGrid& m, int strip, int l) {
+        const int sy = strip / m.strips_x, sxi = strip - sy * m.strips_x;
+        x0 = sxi * m.w;
+        y0 = sy * m.h;
+        hs = p.ny - y0 < m.h ? p.ny - y0 : m.h;
+        first = y0 - (S - 1);
+        const int c = l - (S - 1);
+        const int col = x0 + c;
+        const bool in_w = c >= 0 && c < m.w && col < p.nx;
+        const bool out = EDGE && !p.px && (col < 0 || col >= p.nx);
+        int gx = col;
+        if (out) gx = col < 0 ? 0 : p.nx - 1;
+        else if (col < 0) gx = col + p.nx;
+        else if (col >= p.nx) gx = col % p.nx;
+        kind = (in_w ? 1 : 0) | (out ? 2 : 0);
+        if (EDGE && !p.px && !out) kind |= (gx == 0 ? 4 : 0) | (gx == p.nx - 1 ? 8 : 0);
+        xany = EDGE && !p.px && (x0 <= S - 1 || x0 - (S - 1) + kMarchLanes >= p.nx);
+        oc = uint32_t(gx);
+        om = uint32_t(gx == 0 ? (p.px ? p.nx - 1 : 0) : gx - 1);
+        op = uint32_t(gx == p.nx - 1 ? (p.px ? 0 : gx) : gx + 1);
+        om1 = row_off(p, first - 1);
+        o0 = row_off(p, first);
+        op1 = row_off(p, first + 1);
+        od = uint32_t(y0) * uint32_t(p.nx);
+        rows = MarchRows{0, 0, 0, 0};
+        fl = 0;
+        fln = 0;
+#pragma unroll
+        for (int q = 0; q < Q; q++) g[q] = gn[q] = wgt(q);
+#pragma unroll
+        for (int k = 0; k < S; k++) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) up2[k][j] = up1[k][j] = mid1[k][j] = 0.0f;
+            fx[k] = fy[k] = 0.0f;
+        }
+        fxn = fyn = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 3; j++) sx[0][j] = sx[1][j] = sxn[0][j] = sxn[1][j] = 0.0f;
+    }
+
+    // Lane l's bits of the row masks: row first + l. Straight walls are nearly all flagged nodes
+    // of a run, and the general path (patch(), then the functor) costs a wavefront some 250
+    // instructions per stage and row: on the 1024^2 cavity the strips along the walls took twice
+    // as long as the others and set the launch time. A straight wall replaces the three
+    // populations it sends back and never reads the unstreamed slots.
+    struct Found {
+        bool special, straight, moving, flag;
+    };
+    LBM_HD Found look(const StepParams& p, const MarchGrid& m, int l) const {
+        Found f{false, false, false, false};
+        if (!EDGE || l >= iterations()) return f;
+        const int r = first + l;
+        if (!row_in(p, r)) {
+            f.special = true;
+            return f;
+        }
+        const int rw = row_at(p, r);
+        const bool edge = !p.py && (rw == 0 || rw == p.ny - 1);
+        if (m.row_info) {
+            const uint8_t info = m.row_info[rw], rc = info & 3;
+            const bool has0 = x0 <= S - 1, has1 = x0 - (S - 1) + kMarchLanes >= p.nx;
+            if (edge && !has0 && !has1) {
+                f.moving = (info & 32) != 0;
+                f.straight = f.moving || (info & 16);
+            } else if (!edge && xany && rc == 1) {
+                f.straight = (!has0 || (info & 4)) && (!has1 || (info & 8));
+            }
+            f.flag = !f.straight && (rc == 2 || (rc == 1 && (has0 || has1)));
+        }
+        f.special = edge || xany || f.flag;
+        return f;
+    }
+
+    // Load what stage 0 of row first + i needs into the next-row registers: the nine pulls (a
+    // source outside the domain reads some node inside it, patch() replaces the value), on x
+    // edges the slots patch() takes (stage 0's of this row from the edge store, state t-1; stage
+    // 1's of the row below from the source, state t), the flags, the force.
+    LBM_HD void prefetch(const StepParams& p, int i) {
+        const Buf src(p.src);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const uint32_t row = CY[q] > 0 ? om1 : (CY[q] < 0 ? op1 : o0);
+            const uint32_t x = CX[q] > 0 ? om : (CX[q] < 0 ? op : oc);
+            gn[q] = St::dec1(src.ld(x, q * p.plane + row), q, p.rho0);
+        }
+        if (FORCED == 2) {
+            const PopBuf<float, true> ff(p.force_field);
+            fxn = ff.ld(2u * oc, 2ll * o0);
+            fyn = ff.ld(2u * oc + 1u, 2ll * o0);
+        }
+        if (EDGE && bit(rows.special & ~(rows.straight & (i > 0 ? rows.straight << 1 : ~0ull)), i)) prefetch_edge(p, i);
+        om1 = o0;
+        o0 = op1;
+        op1 = row_off(p, first + i + 2);
+    }
+    LBM_HD void prefetch_edge(const StepParams& pp, int i) {
+        const StepParams p = march_cold(pp);
+        const int r = first + i;
+        fln = uint32_t(LBM_FLUID);
+        if (bit(rows.flag, i) && !dead()) fln = p.flags[o0 + oc];
+        if (!xany) return;
+        const Buf src(p.src), prev(p.edge_prev);
+        const uint32_t below = row_off(p, r - 1);
+#pragma unroll
+        for (int side = 0; side < 2; side++) {
+            if (side == 0 ? !exl() : !exr()) continue;
+            if (row_in(p, r) && !bit(rows.straight, i)) {
+                const int slot = (p.py ? 0 : 2 * p.nx) + (side == 0 ? 0 : p.ny) + row_at(p, r);
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const int q = march_xq(side, j);
+                    sxn[0][j] = St::dec1(prev.ld(0u, q * (long long)p.n_edge + slot), q, p.rho0);
+                }
+            }
+            if (i > 0 && row_in(p, r - 1) && !bit(rows.straight, i - 1)) {
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const int q = march_xq(side, j);
+                    sxn[1][j] = St::dec1(src.ld(oc, q * p.plane + below), q, p.rho0);
+                }
+            }
+        }
+    }
+
+    // Start iteration i: the loaded row becomes stage 0's, the delayed flags and forces move on.
+    LBM_HD void advance() {
+#pragma unroll
+        for (int q = 0; q < Q; q++) g[q] = gn[q];
+        if (EDGE) {
+            fl = (fl << 8) | fln;
+            fln = 0;
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                sx[0][j] = sxn[0][j];
+                sx[1][j] = sxn[1][j];
+            }
+        }
+        if (FORCED == 2) {
+#pragma unroll
+            for (int k = S - 1; k > 0; k--) {
+                fx[k] = fx[k - 1];
+                fy[k] = fy[k - 1];
+            }
+            fx[0] = fxn;
+            fy[0] = fyn;
+        }
+    }
+
+    // Unstreamed slots of stage k's row r (in the domain; an edge row, or the strip has an x
+    // edge): see the file comment.
+    template <int k>
+    LBM_HD void patch(const StepParams& p, const MarchHist<S>* h, int i, int r, int l) {
+        const bool yl = !p.py && r == 0, yh = !p.py && r == p.ny - 1;
+        if (xany && (exl() || exr())) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const float v = k < 2 ? sx[k < 2 ? k : 0][j] : h->x[k >= 2 ? k - 2 : 0][(i - k) % 3][exl() ? 0 : 1][j];
+                g[march_xq(0, j)] = exl() ? v : g[march_xq(0, j)];
+                g[march_xq(1, j)] = exl() ? g[march_xq(1, j)] : v;
+            }
+        }
+        if ((yl || yh) && !dead()) {
+            const Buf src(p.src), prev(p.edge_prev);
+#pragma unroll
+            for (int s = 0; s < 2; s++) {
+                if (s == 0 ? !yl : !yh) continue;
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const int q = march_yq(s, j);
+                    if (k == 0) g[q] = St::dec1(prev.ld(oc, q * (long long)p.n_edge + (s == 0 ? 0 : p.nx)), q, p.rho0);
+                    else if (k == 1) g[q] = St::dec1(src.ld(oc, q * p.plane + (long long)r * p.nx), q, p.rho0);
+                    else g[q] = h->y[k >= 2 ? k - 2 : 0][s][j][l];
+                }
+            }
+        }
+    }
+
+    // Straight walls: the populations a wall sends back (bc_bounce_back away from corners).
+    LBM_HD void back_x() {
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const int a = march_xq(0, j), b = march_xq(1, j);
+            const float va = g[OPP[a]], vb = g[OPP[b]];
+            g[a] = exl() ? va : g[a];
+            g[b] = exr() ? vb : g[b];
+        }
+    }
+    LBM_HD void back_y(const StepParams& p, bool top, bool moving) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            if ((s == 1) != top) continue;
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                const int q = march_yq(s, j), i = OPP[q];
+                float v = g[i];
+                if (moving) v = v - 6.0f * wgt(i) * p.rho0 * (float(CX[i]) * p.wall_ux + float(CY[i]) * p.wall_uy);
+                g[q] = v;
+            }
+        }
+    }
+
+    // The boundary functors a marching launch covers (march_flag): those that need few registers.
+    LBM_HD void functor(const StepParams& p, uint8_t f, int x, int y) {
+        const Geom G{p.nx, p.ny, p.px, p.py};
+        if (f == LBM_BOUNCE_BACK || f == LBM_MOVING_WALL_BOUNCE_BACK) {
+            bc_bounce_back(g, x, y, G, f == LBM_MOVING_WALL_BOUNCE_BACK, p.wall_ux, p.wall_uy, p.rho0);
+        } else if (f == LBM_ZOU_HE_TOP) {
+            bc_zou_he_top(g, p.u_lid);
+        } else if (f == LBM_ZOU_HE_LEFT) {
+            bc_zou_he_left(g, p.u_lid, (p.quirks & LBM_QUIRK_ZOUHE_RHO) != 0);
+        } else if (f == LBM_CYLINDER) {
+            bc_cylinder(g);
+        }
+    }
+
+    // Before the collision of stage k on a special row of the domain that is no straight wall.
+    template <int k>
+    LBM_HD void before(const StepParams& pp, const MarchHist<S>* h, int i, int l) {
+        const StepParams p = march_cold(pp);
+        const int rw = row_at(p, first + i - k);
+        const bool edge = !p.py && (rw == 0 || rw == p.ny - 1);
+        if (xany || edge) patch<k>(p, h, i, rw, l);
+        if (bit(rows.flag, i - k)) {
+            const uint8_t f = uint8_t(fl >> (8 * k));
+            if (f != LBM_FLUID) functor(p, f, int(oc), rw);
+        }
+    }
+
+    // After the collision of stage k on a special row of the domain: the edge store, the history.
+    template <int k>
+    LBM_HD void after(const StepParams& pp, MarchHist<S>* h, int i, int l, const T* e) {
+        const StepParams p = march_cold(pp);
+        const int r = first + i - k, rw = row_at(p, r);
+        const bool edge = !p.py && (rw == 0 || rw == p.ny - 1);
+        if ((MODE == 1 ? k == 0 : k == S - 2) && own() && r >= y0 && r < y0 + hs && (edge || xany)) {
+            // row slots first, then column slots (edge_slot); a corner fills both
+            const int cols = p.py ? 0 : 2 * p.nx;
+            const int slots[3] = {rw == 0 ? 0 : p.nx, cols + rw, cols + p.ny + rw};
+            const Buf next(p.edge_next), src(p.src);
+#pragma unroll
+            for (int s = 0; s < 3; s++) {
+                if (s == 0 ? !edge : (s == 1 ? !exl() : !exr())) continue;
+#pragma unroll
+                for (int q = 0; q < Q; q++)  // MODE 1: the next unstreamed slots hold this launch's source state
+                    next.st(s == 0 ? oc : 0u, q * (long long)p.n_edge + slots[s],
+                            MODE == 1 ? src.ld(oc, q * p.plane + (long long)rw * p.nx) : e[q]);
+            }
+        }
+        if (k <= S - 3 && !bit(rows.straight, i - k)) {
+            constexpr int kk = k < MarchHist<S>::K ? k : 0;
+            if (xany && (exl() || exr())) {
+#pragma unroll
+                for (int j = 0; j < 3; j++) h->x[kk][(i - k) % 3][exl() ? 0 : 1][j] = exl() ? g[march_xq(0, j)] : g[march_xq(1, j)];
+            }
+            if (edge) {
+                const int s = rw == 0 ? 0 : 1;
+#pragma unroll
+                for (int j = 0; j < 3; j++) h->y[kk][s][j][l] = s == 0 ? g[march_yq(0, j)] : g[march_yq(1, j)];
+            }
+        }
+    }
+
+    // Stage k of iteration i (i >= 2k) on g: boundaries, collision, and what the stage leaves
+    // behind. MODE 1's stage 1 sums moments.
+    template <int k>
+    LBM_HD void stage(const StepParams& p, const MarchGrid& m, MarchHist<S>* h, int i, int l, MomAcc& acc) {
+        const bool special = EDGE && bit(rows.special, i - k);
+        const bool wall = EDGE && bit(rows.straight, i - k);
+        if (special) {
+            if (wall) {
+                if (xany) back_x();
+                else back_y(p, first + i - k > 0, bit(rows.moving, i - k));
+            } else {
+                if (!row_in(p, first + i - k)) return;
+                before<k>(p, h, i, l);
+            }
+        }
+        // Opaque from here: the compiler would otherwise lay out the collision twice, once per outcome.
+        int saves = special && (MODE == 1 || !wall || p.edge_all);
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (EDGE) {
+            saves = __builtin_amdgcn_readfirstlane(saves);
+            asm volatile("" : "+s"(saves));
+        }
+#endif
+        const float Fx = FORCED == 2 ? fx[k] : (FORCED ? p.fx : 0.0f), Fy = FORCED == 2 ? fy[k] : (FORCED ? p.fy : 0.0f);
+        const Macro mc = FORCED ? macroscopics(g, Fx, Fy) : macroscopics_unforced(g);
+        if (MODE == 1 && k == 1) {  // only rows y0 .. y0 + hs - 1 get here
+            if (own()) {
+                acc.rho += double(mc.rho);
+                acc.jmag += double(mc.rho * sqrtf(mc.ux * mc.ux + mc.uy * mc.uy));
+                acc.pimag += double(pi_magnitude(g));
+            }
+            return;
+        }
+        const bool rows45 = (p.quirks & LBM_QUIRK_MRT_FORCE_ROWS) != 0;
+        if (COLL == LBM_BGK) collide_bgk(g, mc, Fx, Fy, p.omega, FORCED != 0);
+        else if (COLL == kMarchMrtCons) collide_mrt_t<true>(g, mc, Fx, Fy, p.S, rows45, FORCED != 0);
+        else if (COLL == LBM_MRT) collide_mrt_t<false>(g, mc, Fx, Fy, p.S, rows45, FORCED != 0);
+        else collide_cm(g, mc, Fx, Fy, p.S, MODE == 1 ? p.avg : nullptr);
+        constexpr bool out = MODE == 1 ? k == 0 : k == S - 1;
+        T e[Q];
+#pragma unroll
+        for (int q = 0; q < Q; q++) e[q] = St::enc1(g[q], q, p.rho0);
+        // the last stage is only reached on the strip's own rows; MODE 1's stage 0 has a halo row
+        // on either side
+        const bool own_row = MODE == 1 ? (i >= 1 && i <= hs) : true;
+        if (out && own_row) {
+            if (own()) {
+                const Buf dst(p.dst);
+#pragma unroll
+                for (int q = 0; q < Q; q++) dst.st(oc, q * p.plane + od, e[q]);
+                if (p.out_rho) {
+                    const PopBuf<float, true> r(p.out_rho), u(p.out_ux), v(p.out_uy);
+                    r.st(oc, od, mc.rho);
+                    u.st(oc, od, mc.ux);
+                    v.st(oc, od, mc.uy);
+                }
+            }
+            od += uint32_t(p.nx);
+        }
+        if (MODE == 2 && !out) {
+            const int r = first + i - k;
+            if (own() && r >= y0 && r < y0 + hs) {
+                const Buf mid(static_cast<const char*>(p.mid) + k * m.mid_stride * B);
+#pragma unroll
+                for (int q = 0; q < Q; q++) mid.st(oc, q * p.plane + (long long)r * p.nx, e[q]);
+            }
+        }
+        if (STORE != LBM_F32 && !(out && MODE != 1)) {  // later stages read what a one-step launch would have stored
+#pragma unroll
+            for (int q = 0; q < Q; q++) g[q] = St::dec1(e[q], q, p.rho0);
+        }
+        // straight walls read no unstreamed slot, so their edge nodes are only saved for whatever
+        // runs after the last marching launch of a call
+        if (EDGE && k <= S - 2 && saves) after<k>(p, h, i, l, e);
+    }
+
+    // Hand stage k's row to stage k+1: `a` = populations 1, 5, 8 of the lane to the left, `b` =
+    // 3, 6, 7 of the lane to the right; g becomes the pull of the row below.
+    template <int k>
+    LBM_HD void hand_over(const float* a, const float* b) {
+        const float n0 = g[0], n2 = g[2];
+        g[0] = mid1[k][0];
+        g[1] = mid1[k][1];
+        g[3] = mid1[k][2];
+        g[2] = up2[k][0];
+        g[5] = up2[k][1];
+        g[6] = up2[k][2];
+        g[7] = b[2];
+        g[8] = a[2];
+        mid1[k][0] = n0;
+        mid1[k][1] = a[0];
+        mid1[k][2] = b[0];
+#pragma unroll
+        for (int j = 0; j < 3; j++) up2[k][j] = up1[k][j];
+        up1[k][0] = n2;
+        up1[k][1] = a[1];
+        up1[k][2] = b[1];
+    }
+};
+
+}  // namespace lbm

@@ -1,0 +1,10 @@
+// lbm_march_bf16.hip — the marching multi-step kernels, bf16 storage.
+#include "lbm_march_kernels.hpp"
+
+namespace lbm {
+
+hipError_t launch_march_bf16(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s) {
+    return launch_march_s<LBM_BF16_SHIFTED>(coll, steps, p, m, edge, wide, s);
+}
+
+}  // namespace lbm

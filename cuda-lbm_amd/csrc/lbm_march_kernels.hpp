@@ -1,0 +1,126 @@
+// lbm_march_kernels.hpp — gfx950 kernels of lbm_march.hpp; included by one .hip per storage
+// format (they compile side by side).
+#pragma once
+
+#include "lbm_kernels.hpp"
+#include "lbm_march.hpp"
+
+#include <utility>
+
+namespace lbm {
+
+// Lane l's value from lane l - 1 / l + 1 of the wavefront (DPP wave shifts; the end lanes get 0).
+__device__ __forceinline__ float lane_left(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_right(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x130, 0xf, 0xf, true));
+}
+
+template <int k, int S, class L>
+__device__ __forceinline__ void march_stage(L& w, const StepParams& p, const MarchGrid& m, MarchHist<S>* h, int i, int l,
+                                            MomAcc& acc) {
+    if (i < 2 * k) return;  // the rows this stage needs are still on their way up
+    w.template stage<k>(p, m, h, i, l, acc);
+    if constexpr (k < S - 1) {
+        const float a[3] = {lane_left(w.g[1]), lane_left(w.g[5]), lane_left(w.g[8])};
+        const float b[3] = {lane_right(w.g[3]), lane_right(w.g[6]), lane_right(w.g[7])};
+        w.template hand_over<k>(a, b);
+    }
+}
+template <int S, class L, int... ks>
+__device__ __forceinline__ void march_stages(L& w, const StepParams& p, const MarchGrid& m, MarchHist<S>* h, int i, int l,
+                                             MomAcc& acc, std::integer_sequence<int, ks...>) {
+    (march_stage<ks, S>(w, p, m, h, i, l, acc), ...);
+}
+
+template <int COLL, int STORE, int S, bool EDGE, int FORCED, int MODE>
+__device__ __forceinline__ void march_run(MarchLane<COLL, STORE, S, EDGE, FORCED, MODE>& w, const StepParams& p,
+                                          const MarchGrid& m, MarchHist<S>* h, int l, MomAcc& acc) {
+    const int n = w.iterations();
+    if (EDGE) {
+        const auto f = w.look(p, m, l);
+        w.rows = MarchRows{__builtin_amdgcn_ballot_w64(f.special), __builtin_amdgcn_ballot_w64(f.straight),
+                           __builtin_amdgcn_ballot_w64(f.moving), __builtin_amdgcn_ballot_w64(f.flag)};
+    }
+    w.prefetch(p, 0);
+    for (int i = 0; i < n; i++) {
+        if (EDGE) {  // opaque per iteration: no second copy of the march for strips without an x edge
+            w.xany = __builtin_amdgcn_readfirstlane(w.xany);
+            asm volatile("" : "+s"(w.xany));
+        }
+        w.advance();
+        if (i + 1 < n) w.prefetch(p, i + 1);
+        __builtin_amdgcn_sched_barrier(0);  // the next row's loads are issued before this row's work
+        march_stages<S>(w, p, m, h, i, l, acc, std::make_integer_sequence<int, S>{});
+    }
+}
+
+// WGW wavefronts per workgroup: neighbours along x, so that they start together and the cache
+// lines their strips share are in one L2 at one time. No wavefront waits for another.
+template <int COLL, int STORE, int S, bool EDGE, int FORCED, int MODE, int WGW>
+__global__ __launch_bounds__(kMarchLanes * WGW) void march_kernel(StepParams p, MarchGrid m, int nb, double* partials) {
+    __shared__ MarchHist<S> hist[EDGE && S > 2 ? WGW : 1];
+    const int per = nb / kXcds;
+    const int lb = (int(blockIdx.x) % kXcds) * per + int(blockIdx.x) / kXcds;
+    const int wv = __builtin_amdgcn_readfirstlane(int(threadIdx.x / kMarchLanes));
+    const int strip = lb * WGW + wv;
+    if (strip >= m.n_strips) return;
+    const int l = int(threadIdx.x % kMarchLanes);
+    MomAcc acc{0.0, 0.0, 0.0};
+    MarchLane<COLL, STORE, S, EDGE, FORCED, MODE> w;
+    w.init(p, m, strip, l);
+    march_run(w, p, m, &hist[EDGE && S > 2 ? wv : 0], l, acc);
+    if constexpr (MODE == 1) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            acc.rho += __shfl_xor(acc.rho, off, 64);
+            acc.jmag += __shfl_xor(acc.jmag, off, 64);
+            acc.pimag += __shfl_xor(acc.pimag, off, 64);
+        }
+        if (l == 0) {
+            partials[3 * (long long)strip + 0] = acc.rho;
+            partials[3 * (long long)strip + 1] = acc.jmag;
+            partials[3 * (long long)strip + 2] = acc.pimag;
+        }
+    }
+}
+
+template <int COLL, int STORE, int S, bool EDGE, int FORCED, int MODE, int WGW>
+hipError_t launch_march_t(const StepParams& p, const MarchGrid& m, double* partials, hipStream_t s) {
+    const int wgs = (m.n_strips + WGW - 1) / WGW, nb = (wgs + kXcds - 1) / kXcds * kXcds;
+    hipLaunchKernelGGL((march_kernel<COLL, STORE, S, EDGE, FORCED, MODE, WGW>), dim3(unsigned(nb)), dim3(kMarchLanes * WGW), 0, s,
+                       p, m, nb, partials);
+    return hipGetLastError();
+}
+
+template <int COLL, int STORE, int S, bool EDGE, int MODE>
+hipError_t launch_march_f(const StepParams& p, const MarchGrid& m, bool wide, double* partials, hipStream_t s) {
+    const int forced = p.force_field ? 2 : (p.forced ? 1 : 0);
+    if (forced == 2) return wide ? launch_march_t<COLL, STORE, S, EDGE, 2, MODE, 4>(p, m, partials, s) : launch_march_t<COLL, STORE, S, EDGE, 2, MODE, 1>(p, m, partials, s);
+    if (forced == 1) return wide ? launch_march_t<COLL, STORE, S, EDGE, 1, MODE, 4>(p, m, partials, s) : launch_march_t<COLL, STORE, S, EDGE, 1, MODE, 1>(p, m, partials, s);
+    return wide ? launch_march_t<COLL, STORE, S, EDGE, 0, MODE, 4>(p, m, partials, s) : launch_march_t<COLL, STORE, S, EDGE, 0, MODE, 1>(p, m, partials, s);
+}
+template <int COLL, int STORE, int S, int MODE>
+hipError_t launch_march_v(const StepParams& p, const MarchGrid& m, bool edge, bool wide, double* partials, hipStream_t s) {
+    return edge ? launch_march_f<COLL, STORE, S, true, MODE>(p, m, wide, partials, s) : launch_march_f<COLL, STORE, S, false, MODE>(p, m, wide, partials, s);
+}
+
+// The S instances of one storage format: 4, and 6 in single precision.
+template <int STORE, int S>
+hipError_t launch_march_c(int coll, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s) {
+    if (coll == LBM_BGK) return launch_march_v<LBM_BGK, STORE, S, 0>(p, m, edge, wide, nullptr, s);
+    if (coll == LBM_CM) return launch_march_v<LBM_CM, STORE, S, 0>(p, m, edge, wide, nullptr, s);
+    if (p.S[0] == 0.0f && p.S[3] == 0.0f && p.S[5] == 0.0f)
+        return launch_march_v<kMarchMrtCons, STORE, S, 0>(p, m, edge, wide, nullptr, s);
+    return launch_march_v<LBM_MRT, STORE, S, 0>(p, m, edge, wide, nullptr, s);
+}
+template <int STORE>
+hipError_t launch_march_s(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s) {
+    if (steps == 4) return launch_march_c<STORE, 4>(coll, p, m, edge, wide, s);
+    if constexpr (STORE == LBM_F32)
+        if (steps == 6) return launch_march_c<STORE, 6>(coll, p, m, edge, wide, s);
+    return hipErrorInvalidValue;
+}
+
+}  // namespace lbm

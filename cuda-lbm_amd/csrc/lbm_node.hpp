@@ -62,6 +62,15 @@ LBM_HD Macro macroscopics(const float* g, float fx, float fy) {
     return m;
 }
 
+// macroscopics() without a force (the half-force adds, exact zeros then, left out).
+LBM_HD Macro macroscopics_unforced(const float* g) {
+    const float r = (((((((g[0] + g[1]) + g[2]) + g[3]) + g[4]) + g[5]) + g[6]) + g[7]) + g[8];
+    const float jx = ((((g[1] - g[3]) + g[5]) - g[6]) - g[7]) + g[8];
+    const float jy = ((((g[2] - g[4]) + g[5]) + g[6]) - g[7]) - g[8];
+    const float inv = recip(r);
+    return Macro{r, jx * inv, jy * inv};
+}
+
 // Raw second-moment magnitude |Pi| = sqrt(Pxx^2 + 2Pxy^2 + Pyy^2) (macroscopics.cu:24-32).
 LBM_HD float pi_magnitude(const float* g) {
     float d = g[5] + g[6] + g[7] + g[8];

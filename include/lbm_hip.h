@@ -105,9 +105,9 @@ typedef struct lbm_config {
     float    wall_u[2];      /* velocity of LBM_MOVING_WALL_BOUNCE_BACK nodes               */
     float    u_lid;          /* Scenario::u_max as used by REGULARIZED_INLET_TOP / ZOU_HE_*  */
     uint32_t quirks;         /* LBM_QUIRK_* bitmask                                         */
-    int32_t  steps_per_launch; /* 0: two time steps per launch wherever supported (the same
-                                  algorithm; agrees with 1 to FP32 rounding), 1: one step per
-                                  launch                                                       */
+    int32_t  steps_per_launch; /* 0: two or more time steps per launch wherever supported (the
+                                  same algorithm; agrees with 1 to FP32 rounding), 1: one step
+                                  per launch                                                   */
     int32_t  reserved[7];
 } lbm_config;
 
@@ -143,14 +143,15 @@ int lbm_set_force_field(lbm_ctx* ctx, const float* force, int on_device);
 /* One call = `nsteps` iterations of the reference's loop body (main.cu:96-114):
  * stream, boundaries, macroscopics, forces, IBM, Guo correction, equilibrium, collision,
  * fused into one pull-scheme kernel per step (plus the IBM / adapter passes when active),
- * or into one kernel per pair of steps where steps_per_launch allows it (an odd remainder
- * runs as a single step). Asynchronous on the context's stream. The last step also stores
+ * or into one kernel per two, four or six steps where steps_per_launch allows it (an odd
+ * remainder runs as a single step). Asynchronous on the context's stream. The last step also stores
  * rho and u. */
 int lbm_step(lbm_ctx* ctx, int32_t nsteps);
 int lbm_sync(lbm_ctx* ctx);
 int lbm_get_timestep(const lbm_ctx* ctx, int64_t* t);
 /* Time steps per kernel launch that lbm_step uses for the current configuration, flags and
- * bodies: 2 (two-step launches) or 1. No counterpart in the reference, which launches eight
+ * bodies: 2 (several steps per launch: two, or four or six on the grids where that is faster)
+ * or 1. No counterpart in the reference, which launches eight
  * kernels per step; for profiling and bandwidth accounting. */
 int lbm_get_steps_per_launch(const lbm_ctx* ctx, int32_t* steps);
 

@@ -1,0 +1,132 @@
+"""Marching multi-step launches (lbm_march.hpp): every form against one step per launch.
+
+On the CPU the host emulation runs the kernel's lane body, 64 lanes in lockstep; both sides run
+the same arithmetic per node, so the populations are equal bit for bit. On the GPU the kernels
+contract multiply-adds differently: there the bound is the one of the two-step launches."""
+import numpy as np
+import pytest
+
+from helpers import layout_case, max_rel, run_emu, run_gpu
+from lbm_amd import _abi as A
+
+LAYOUTS = ["periodic", "channel", "cavity_mw", "zouhe_top", "open"]  # those whose functors are local
+# steps, columns and rows per strip: the widest strip of each form, the aligned one, and strips
+# narrower and shorter than their halo; heights that leave one-row remainders
+FORMS = [(4, 58, 8), (4, 7, 2), (4, 48, 12), (6, 54, 16), (6, 48, 52), (6, 9, 3)]
+
+
+def _code(form):
+    s, w, h = form
+    return 1000000 * s + 1000 * w + h
+
+
+@pytest.mark.parametrize("form", FORMS, ids=lambda f: "s%dw%dh%d" % f)
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("coll", [A.LBM_BGK, A.LBM_MRT, A.LBM_CM], ids=["bgk", "mrt", "cm"])
+def test_emulated_march_equals_one_step_launches(coll, layout, form):
+    # 13 steps: marching launches, a two-step remainder, an odd one; 150 columns give strips that
+    # touch the left edge, no edge, the right edge
+    case = layout_case(layout, 150, 37, coll, forced=form[0] == 4)
+    f1, r1, u1, _ = run_emu(case, 13, seg=1)
+    f2, r2, u2, _ = run_emu(case, 13, two_ty=_code(form))
+    f3, r3, u3, _ = run_emu(case, 12, two_ty=_code(form), reverse=True)
+    f4, r4, u4, _ = run_emu(case, 12, seg=1)
+    assert np.array_equal(f1, f2) and np.array_equal(r1, r2) and np.array_equal(u1, u2)
+    assert np.array_equal(f3, f4) and np.array_equal(r3, r4) and np.array_equal(u3, u4)
+
+
+@pytest.mark.parametrize("nx,ny", [(16, 16), (17, 40), (64, 18), (70, 16), (130, 64)])
+@pytest.mark.parametrize("layout", ["periodic", "channel", "cavity_mw", "open"])
+def test_emulated_march_small_and_ragged_grids(layout, nx, ny):
+    case = layout_case(layout, nx, ny, A.LBM_BGK)
+    f1, *_ = run_emu(case, 12, seg=1)
+    for form in ((4, 58, 5), (6, 54, 11), (6, 48, 52)):
+        f2, *_ = run_emu(case, 12, two_ty=_code(form))
+        assert np.array_equal(f1, f2), form
+
+
+@pytest.mark.parametrize("storage", [A.LBM_F16_SHIFTED, A.LBM_BF16_SHIFTED], ids=["f16", "bf16"])
+@pytest.mark.parametrize("layout", ["periodic", "cavity_mw", "open"])
+def test_emulated_march_reduced_storage_and_force_field(storage, layout):
+    case = layout_case(layout, 150, 37, A.LBM_MRT, storage=storage)
+    rng = np.random.default_rng(3)
+    case.force_field = (1e-5 * rng.standard_normal((37, 150, 2))).astype(np.float32)
+    f1, *_ = run_emu(case, 8, seg=2)
+    f2, *_ = run_emu(case, 8, two_ty=_code((4, 58, 9)))
+    assert np.array_equal(f1, f2)
+
+
+def test_emulated_march_inner_flags():
+    # solid nodes inside the grid (class 2 rows), on strip borders and next to the walls
+    case = layout_case("cavity_mw", 150, 37, A.LBM_CM)
+    case.flags[1:4, 1:5] = A.CYLINDER
+    case.flags[17:20, 56:60] = A.CYLINDER
+    case.flags[35, 148] = A.BOUNCE_BACK
+    f1, *_ = run_emu(case, 12, seg=1)
+    for form in ((4, 58, 8), (6, 54, 16)):
+        f2, *_ = run_emu(case, 12, two_ty=_code(form))
+        assert np.array_equal(f1, f2), form
+
+
+# grids that take each marching form of the library: four and six steps, with and without edges,
+# narrow and wide workgroups; 13 steps also run a remainder
+GPU_GRIDS = [("periodic", 1030, 900), ("cavity_mw", 1030, 900), ("channel", 1016, 911), ("zouhe_top", 1001, 910),
+             ("open", 1001, 910), ("periodic", 2600, 2100), ("periodic", 2608, 3300), ("cavity_mw", 3100, 2750),
+             ("open", 3007, 2900)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout,nx,ny", GPU_GRIDS)
+@pytest.mark.parametrize("coll", [A.LBM_BGK, A.LBM_MRT, A.LBM_CM], ids=["bgk", "mrt", "cm"])
+def test_gpu_march_matches_one_step_launches(layout, nx, ny, coll):
+    print(f"case march {layout} {nx}x{ny} coll={coll}", flush=True)
+    case = layout_case(layout, nx, ny, coll, forced=coll != A.LBM_MRT)
+    case.config.steps_per_launch = 1
+    f1, _, u1, s1 = run_gpu(case, 13)
+    s1.close()
+    case.config.steps_per_launch = 0
+    f2, _, u2, s2 = run_gpu(case, 13)
+    s2.close()
+    # contraction differs between the kernels: FP32 rounding (as for the two-step launches)
+    assert max_rel(f2, f1) <= 1e-5 and float(np.max(np.abs(u2 - u1))) <= 1e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage", [A.LBM_F16_SHIFTED, A.LBM_BF16_SHIFTED], ids=["f16", "bf16"])
+@pytest.mark.parametrize("layout", ["periodic", "cavity_mw"])
+def test_gpu_march_reduced_storage_and_force_field(layout, storage):
+    print(f"case march {layout} storage={storage}", flush=True)
+    case = layout_case(layout, 1300, 1300, A.LBM_BGK, storage=storage)
+    rng = np.random.default_rng(3)
+    case.force_field = (1e-5 * rng.standard_normal((1300, 1300, 2))).astype(np.float32)
+    case.config.steps_per_launch = 1
+    f1, *_, s1 = run_gpu(case, 8)
+    s1.close()
+    case.config.steps_per_launch = 0
+    f2, *_, s2 = run_gpu(case, 8)
+    s2.close()
+    quantum = 2.0 ** -11 if storage == A.LBM_F16_SHIFTED else 2.0 ** -8
+    assert float(np.max(np.abs(f2 - f1))) <= 4 * 0.05 * quantum  # a rounding flip of a few deviations
+
+
+@pytest.mark.gpu
+def test_gpu_march_then_other_forms_keep_the_unstreamed_slots():
+    """A run of marching launches hands its edge nodes to the forms that follow it: new flags
+    between two calls (walls opened: their unstreamed slots are read from then on), an odd step,
+    then marching again, against one step per launch throughout."""
+    from lbm_amd import Solver
+
+    out = []
+    for spl in (1, 0):
+        case = layout_case("cavity_mw", 1030, 900, A.LBM_BGK)
+        case.config.steps_per_launch = spl
+        with Solver(case.config) as s:
+            case.apply(s)
+            s.step(8)
+            fl = case.flags.copy()
+            fl[:, 0] = fl[0, :] = A.FLUID
+            s.set_flags(fl)
+            s.step(1)
+            s.step(9)
+            out.append(s.get_pops())
+    assert max_rel(out[1], out[0]) <= 1e-5
