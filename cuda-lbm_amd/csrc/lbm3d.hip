@@ -43,11 +43,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void s
     const long long per = nb / 8;
     const long long L = b < per * 8 ? (b % 8) * per + b / 8 : b;
     int x, y, z;
-    thread_node(p, L, int(threadIdx.x), x, y, z);
-    x += p.ox;
-    y += p.oy;
-    z += p.oz;
-    if (x >= p.xe || y >= p.ye) return;
+    if (GUO == 0 && p.flat) {
+        if (!flat_node(p, L, int(threadIdx.x), x, y, z)) return;
+    } else {
+        thread_node(p, L, int(threadIdx.x), x, y, z);
+        x += p.ox;
+        y += p.oy;
+        z += p.oz;
+        if (x >= p.xe || y >= p.ye) return;
+    }
     if (p.region == 1 && x >= p.rbox[0] && x < p.rbox[1] && y >= p.rbox[2] && y < p.rbox[3] && z >= p.rbox[4] &&
         z < p.rbox[5])
         return;
@@ -431,22 +435,36 @@ int lbm3d_ctx::one_step(bool write_macros) {
     p.guo = has_guo ? 1 : 0;
     p.corner_uz = (cfg.quirks & LBM_QUIRK_CORNER3D_UZ) ? 1 : 0;
     p.stale_rest = (cfg.quirks & LBM_QUIRK_STALE_REST) ? 1 : 0;
-    // Non-temporal stores keep the written populations from evicting the pulls' shared lines
-    // once the two buffers no longer stay in the 256 MB Infinity Cache (+2% FP32, +4% FP16 at
-    // 256^3); on resident grids they push every write to HBM (-20% FP32 at 64^3 and 96^3).
-    // The switch sits at kNtBufferBytes, three quarters of the cache (the 2-D kernels' cache
-    // threshold too), leaving room for the flags and the other data a step touches; grids
-    // between it and the full cache (about 97^3-105^3 FP32, 122^3-133^3 FP16) were not timed
-    // separately.
-    constexpr double kNtBufferBytes = 192.0e6;
-    p.nt = 2.0 * Q * double(plane) * double(elem_bytes(cfg.storage)) > kNtBufferBytes ? 1 : 0;
     p.wx = wave_cols(cfg.nx);
     p.nbx = (cfg.nx + 64 * p.wx - 1) / (64 * p.wx);
     p.nby = (cfg.ny + 4 / p.wx - 1) / (4 / p.wx);
     p.xe = cfg.nx;
     p.ye = cfg.ny;
     p.nzl = cfg.nz;
-    const long long nblk = (long long)p.nbx * p.nby * cfg.nz;
+    // The launch's nodes: flat, 64 consecutive nodes of the grid per wavefront whatever the row
+    // length, for grids whose functors read no neighbour (the others rely on a wavefront holding
+    // one 64-column group of a row, see needs_pre_launch; a split step needs the box rows). Every
+    // store is then 64 whole aligned elements and no lane idles at row ends. Against a row of
+    // workgroups per grid row, us per step: 250x201x150 MRT F16 324 -> 179, F32 509 -> 319,
+    // 130^3 F32 145 -> 92, 70^3 F16 15.8 -> 11.2, duct 250x128x96 F32 211 -> 143; rows of whole
+    // lines (256, 128, 64) are within 2 % either way.
+    p.flat = !has_guo && !has_reg && !(ibm.active && ibm.split_ok) ? 1 : 0;
+    // Non-temporal stores keep the written populations from evicting the pulls' shared lines
+    // once the two buffers do not fit the 256 MiB Infinity Cache (256^3 F16 382 -> 369, F32 +2 %);
+    // on resident grids they push every write to HBM (us per step without / with: 100^3 CM F32,
+    // 216 MB, 34 / 43; 128^3 F16, 226 MB, 40 / 50; duct 250x128x96 F16, 332 MB, 75 / 75; 64^3 F32
+    // 11 / 13). Stores that do not start on a line write it in parts, which costs more than the
+    // cached lines gain (tunnel 250x128x96 F32 206 / 230): then only flat launches use them.
+    constexpr double kNtBufferBytes = 268.0e6;
+    const bool lines = p.flat || (long long)cfg.nx * (long long)elem_bytes(cfg.storage) % 128 == 0;
+    p.nt = lines && 2.0 * Q * double(plane) * double(elem_bytes(cfg.storage)) > kNtBufferBytes ? 1 : 0;
+    if (p.flat) {
+        magic_div(uint32_t(cfg.nx), p.div_x, p.shift_x);
+        magic_div(uint32_t(cfg.ny), p.div_y, p.shift_y);
+        p.nbx = int((N + 255) / 256);  // as one row of workgroups
+        p.nby = p.nzl = 1;
+    }
+    const long long nblk = (long long)p.nbx * p.nby * p.nzl;
     if (nblk > 0x7fffffffLL) return fail(LBM_E_INVALID, "grid needs too many workgroups");
     const bool fits = cfg.storage == LBM_F32 ? lbm::buf_fits<float>(Q, plane) : lbm::buf_fits<uint16_t>(Q, plane);
     // IBM split step: the nodes outside the band's box on aux_stream (they read neither the IBM

@@ -57,7 +57,23 @@ struct Step3Params {
     int wx;
     int nbx, nby;
     int ox, oy, oz, xe, ye, nzl;
+    // Flat launches (flat_ok): thread t of workgroup L owns node 256 L + t, its coordinates by
+    // multiplication (MagicDiv of nx and ny); the box fields above are unused.
+    int flat;
+    uint32_t div_x, div_y;
+    int shift_x, shift_y;
 };
+
+// n / d for 0 <= n < 2^31 and a divisor 2 <= d < 2^31 fixed per launch: (n mul) >> (31 + s) with
+// s = ceil(log2 d), mul = ceil(2^(31+s) / d) < 2^32. Exact: mul d - 2^(31+s) < d <= 2^s, so the
+// error term stays below 2^(31+s) for every n < 2^31.
+inline void magic_div(uint32_t d, uint32_t& mul, int& shift) {
+    int s = 1;
+    while ((1ull << s) < d) s++;
+    mul = uint32_t(((1ull << (31 + s)) + d - 1) / d);
+    shift = s - 1;
+}
+LBM3_HD uint32_t div_by(uint32_t n, uint32_t mul, int shift) { return uint32_t((uint64_t(n) * mul) >> 32) >> shift; }
 
 // Workgroup of 256 threads: wx = min(4, ceil(nx/64)) wavefronts along x, so a workgroup holds
 // whole rows up to nx = 256 and the partial cache lines of the x-shifted pulls are shared
@@ -73,6 +89,18 @@ LBM3_HD void thread_node(const Step3Params& p, long long L, int t, int& x, int& 
     const int cols = 64 * p.wx;
     x = bx * cols + t % cols;
     y = by * (4 / p.wx) + t / cols;
+}
+
+// The node of thread t of workgroup L in a flat launch; false past the last node.
+LBM3_HD bool flat_node(const Step3Params& p, long long L, int t, int& x, int& y, int& z) {
+    const long long n = L * 256 + t;
+    if (n >= (long long)p.nx * p.ny * p.nz) return false;
+    const uint32_t row = div_by(uint32_t(n), p.div_x, p.shift_x);
+    x = int(uint32_t(n) - row * uint32_t(p.nx));
+    const uint32_t zz = div_by(row, p.div_y, p.shift_y);
+    y = int(row - zz * uint32_t(p.ny));
+    z = int(zz);
+    return true;
 }
 
 // Population storage: FP32, or FP16/BF16 of the shifted deviation f - w rho0.

@@ -302,6 +302,40 @@ int emu3d_run_ibm(const lbm3d_config* c, const float* f_in, const uint8_t* flags
 
 }  // extern "C"
 
+// The flat launch's node mapping over a whole grid: every node once, in order, with its
+// coordinates, and no thread of the last workgroup past the grid. 0 when it holds.
+extern "C" int emu3_flat_check(int nx, int ny, int nz) {
+    Step3Params p{};
+    p.nx = nx;
+    p.ny = ny;
+    p.nz = nz;
+    p.flat = 1;
+    magic_div(uint32_t(nx), p.div_x, p.shift_x);
+    magic_div(uint32_t(ny), p.div_y, p.shift_y);
+    const long long N = (long long)nx * ny * nz;
+    for (long long n = 0; n < (N + 255) / 256 * 256; n++) {
+        int x = -1, y = -1, z = -1;
+        const bool in = flat_node(p, n / 256, int(n % 256), x, y, z);
+        if (in != (n < N)) return 1;
+        if (in && (x != n % nx || y != (n / nx) % ny || z != n / ((long long)nx * ny))) return 2;
+    }
+    return 0;
+}
+// div_by against the integer division for one divisor at the ends of the range and around
+// multiples of the divisor.
+extern "C" int emu3_div_check(uint32_t d) {
+    uint32_t mul;
+    int shift;
+    magic_div(d, mul, shift);
+    const uint32_t top = 0x7fffffffu;
+    for (uint32_t k = 0; k < 20000; k++) {
+        const uint32_t m = uint32_t((uint64_t(top / d) * k) / 19999) * d;
+        for (uint32_t n : {m, m + d - 1, m > 0 ? m - 1 : 0, k, top - k})
+            if (n <= top && div_by(n, mul, shift) != n / d) return 1;
+    }
+    return 0;
+}
+
 #ifdef EMU_MAIN
 // Bounds matrix: every access of the step body and the IBM pass on exact-size buffers under
 // ASan, over grid shapes below, at and above one wavefront row, every periodicity pattern,
