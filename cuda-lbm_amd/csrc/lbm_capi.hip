@@ -189,11 +189,14 @@ int lbm_ctx::ahead_step(bool write_macros) {
     p.edge_prev = d_edge[edge_cur];
     p.edge_next = d_edge[1 - edge_cur];
     p.n_edge = n_edge;
+    MarchPolicy mp;
+    if (flags_march) mp = march_ahead_policy(cfg.nx, cfg.ny, plane, cfg.storage, d_flags || n_edge > 0);
     const Step2Policy lp = ahead_policy(plane, cfg.storage);
-    const long long np = ahead_partials_needed(p, lp);
+    const long long np = mp.steps ? march_strips(p, mp) : ahead_partials_needed(p, lp);
     rc = ensure_partials(np);
     if (rc) return rc;
-    e = launch_step_ahead(cfg.collision, cfg.storage, p, lp, partials, stream);
+    if (mp.steps) e = launch_march_ahead(cfg.storage, p, mp, d_row_info, partials, stream);
+    else e = launch_step_ahead(cfg.collision, cfg.storage, p, lp, partials, stream);
     if (e != hipSuccess) return hip_fail(e, "look-ahead step launch");
     e = launch_finalize_ahead(partials, np, (long long)N, d_ahead, d_ahead64, d_avg, d_avg64, stream);
     if (e != hipSuccess) return hip_fail(e, "finalize launch");

@@ -8,6 +8,9 @@ namespace lbm {
 
 constexpr int kBlock = 256;      // workgroup of the auxiliary kernels (4 wave64)
 constexpr int kMaxStepBlock = 512;
+// The one workgroup that sums a launch's partial triples: its time is the latency of its chain of
+// loads, so all 16 wavefronts (4 300 triples of the 4096 x 1024 channel: 7.2 us with 256 threads).
+constexpr int kFinalBlock = 1024;
 
 // Workgroup i runs on XCD i % 8. With remap, each XCD gets a contiguous run of logical
 // workgroups, so the cache lines that neighbouring row segments share stay in one XCD's L2
@@ -26,7 +29,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // Deterministic block sum of three doubles; result valid in thread 0.
 __device__ __forceinline__ void block_sum3(double& a, double& b, double& c) {
-    __shared__ double part[3][kMaxStepBlock / 64];
+    __shared__ double part[3][kFinalBlock / 64];
     a = wave_sum(a);
     b = wave_sum(b);
     c = wave_sum(c);
@@ -240,14 +243,14 @@ __global__ __launch_bounds__(kBlock) void finalize_avg_kernel(const double* part
 
 // After a look-ahead launch: the averages that launch collided with (`ahead`) become the
 // reported ones (`avg`), and the launch's partial sums become the next step's `ahead`.
-__global__ __launch_bounds__(kBlock) void finalize_ahead_kernel(const double* partials, long long n, double inv_nodes,
+__global__ __launch_bounds__(kFinalBlock) void finalize_ahead_kernel(const double* partials, long long n, double inv_nodes,
                                                               float* ahead, double* ahead64, float* avg, double* avg64) {
     if (threadIdx.x < 3) {
         avg[threadIdx.x] = ahead[threadIdx.x];
         avg64[threadIdx.x] = ahead64[threadIdx.x];
     }
     double a = 0.0, b = 0.0, c = 0.0;
-    for (long long i = threadIdx.x; i < n; i += kBlock) {
+    for (long long i = threadIdx.x; i < n; i += kFinalBlock) {
         a += partials[3 * i];
         b += partials[3 * i + 1];
         c += partials[3 * i + 2];
@@ -569,6 +572,27 @@ Step2Policy step2_policy(long long plane, int storage, int coll) {
     return lp;
 }
 
+// Rows per marching strip. The height balances the halo rows (S - 1 + h per h) against the
+// number of wavefronts: the cost is wavefronts per SIMD, rounded up, times rows, with a penalty
+// for one or two wavefronts per SIMD, which leave the vector ALU idle while they wait.
+static int march_height(int nx, int ny, int w, int steps, bool edge) {
+    const long long sx = (nx + w - 1) / w;
+    const int resident = edge ? 4 : 5;  // wavefronts per SIMD
+    double best = 1e30;
+    int height = 1;
+    for (int h = 1; h <= 48; h++) {
+        const double n = double(sx * ((ny + h - 1) / h)) / double(kSimds), rows = h + steps - 1;
+        const double c = std::ceil(n);
+        const double idle = c <= 1 ? 1.7 : (c <= 2 ? 1.1 : (c <= 3 ? 1.03 : 1.0));
+        const double cost = (c <= resident ? c * idle : n + 0.5) * rows;
+        if (cost < best) {
+            best = cost;
+            height = h;
+        }
+    }
+    return height;
+}
+
 // Measured on MI355X, us per step, 48-step calls, against the two-step forms (tiles or strips)
 // of the same build and box; S x w x h the marching shape:
 //   periodic   64^2 BGK F32  2.41 -> 1.58 (4x58x1)     128^2 2.33 -> 1.71 (4x58x1)
@@ -587,9 +611,6 @@ Step2Policy step2_policy(long long plane, int storage, int coll) {
 // at four steps, by the vector ALU at six), later for CM (more arithmetic) and walled grids.
 // Aligned 48-column strips, four to a workgroup, write whole 64-byte granules and keep the
 // neighbours' shared lines in L2; the 14 % of lanes they idle only pay in HBM and for BGK.
-// The height balances the halo rows (S - 1 + h per h) against the number of wavefronts: the cost
-// is wavefronts per SIMD, rounded up, times rows, with a penalty for one or two wavefronts per
-// SIMD, which leave the vector ALU idle while they wait.
 MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll, bool edge, int steps_left) {
     MarchPolicy lp;
     const bool f32 = storage == LBM_F32;
@@ -609,19 +630,7 @@ MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll,
         }
         return lp;
     }
-    const long long sx = (nx + lp.w - 1) / lp.w;
-    const int resident = edge ? 4 : 5;  // wavefronts per SIMD
-    double best = 1e30;
-    for (int h = 1; h <= 48; h++) {
-        const double n = double(sx * ((ny + h - 1) / h)) / double(kSimds), rows = h + lp.steps - 1;
-        const double c = std::ceil(n);
-        const double idle = c <= 1 ? 1.7 : (c <= 2 ? 1.1 : (c <= 3 ? 1.03 : 1.0));
-        const double cost = (c <= resident ? c * idle : n + 0.5) * rows;
-        if (cost < best) {
-            best = cost;
-            lp.h = h;
-        }
-    }
+    lp.h = march_height(nx, ny, lp.w, lp.steps, edge);
     return lp;
 }
 
@@ -638,6 +647,40 @@ hipError_t launch_march(int coll, int storage, const StepParams& p, const MarchP
     if (storage == LBM_F16_SHIFTED) return launch_march_f16(coll, lp.steps, p, m, edge, lp.wide, s);
     if (storage == LBM_BF16_SHIFTED) return launch_march_bf16(coll, lp.steps, p, m, edge, lp.wide, s);
     return launch_march_f32(coll, lp.steps, p, m, edge, lp.wide, s);
+}
+
+// Measured on MI355X, us per step with the finalize, against the LDS strips: channel 4096x1024
+// F32 97.7 -> 85.2 (h 20..24; 16 104), F16 78.4 -> 65.7; 1024^2 F32 32.4 -> 27.2; 300x200 22.4
+// -> 12.3; 700x500 BF16 56 -> 17.9 (few strips: the LDS form marched 32 rows in each); beyond
+// the cache 6000x3000 F32 359 -> 339 at h 16 (359 at 32).
+MarchPolicy march_ahead_policy(int nx, int ny, long long plane, int storage, bool edge) {
+    MarchPolicy lp;
+    const bool f32 = storage == LBM_F32;
+    if (nx < kMarchMinSide || ny < kMarchMinSide) return lp;
+    if (!(f32 ? buf_fits<float>(Q, plane) : buf_fits<uint16_t>(Q, plane))) return lp;
+    const double bytes = 2.0 * 9.0 * double(plane) * (f32 ? 4.0 : 2.0);
+    lp.steps = 2;
+    lp.w = kMarchLanes - 2;
+    lp.h = bytes > 600.0e6 ? 16 : march_height(nx, ny, lp.w, 2, edge);
+    return lp;
+}
+
+long long march_strips(const StepParams& p, const MarchPolicy& lp) {
+    return (long long)((p.nx + lp.w - 1) / lp.w) * ((p.ny + lp.h - 1) / lp.h);
+}
+
+hipError_t launch_march_ahead(int storage, const StepParams& p, const MarchPolicy& lp, const uint8_t* row_info, double* partials,
+                              hipStream_t s) {
+    if (p.n_edge != edge_count(p.nx, p.ny, p.px, p.py) || !partials || !p.avg) return hipErrorInvalidValue;
+    if (p.n_edge > 0 && (!p.edge_prev || !p.edge_next)) return hipErrorInvalidValue;
+    if (lp.steps != 2 || p.nx < kMarchMinSide || p.ny < kMarchMinSide || lp.w < 1 || lp.w > kMarchLanes - 2 || lp.h < 1 ||
+        lp.h + 2 > kMarchMaxRows || march_strips(p, lp) > 0x7fffff00LL)
+        return hipErrorInvalidValue;
+    const MarchGrid m{(p.nx + lp.w - 1) / lp.w, int(march_strips(p, lp)), lp.w, lp.h, row_info, 0};
+    const bool edge = p.flags || !p.px || !p.py;
+    if (storage == LBM_F16_SHIFTED) return launch_march_ahead_f16(p, m, edge, lp.wide, partials, s);
+    if (storage == LBM_BF16_SHIFTED) return launch_march_ahead_bf16(p, m, edge, lp.wide, partials, s);
+    return launch_march_ahead_f32(p, m, edge, lp.wide, partials, s);
 }
 
 hipError_t launch_edge_copy(int storage, void* buf, void* store, long long plane, int nx, int ny, int px, int py,
@@ -698,7 +741,7 @@ hipError_t launch_step_ahead(int coll, int storage, const StepParams& p, const S
 
 hipError_t launch_finalize_ahead(const double* partials, long long n, long long N, float* ahead, double* ahead64, float* avg,
                                  double* avg64, hipStream_t s) {
-    hipLaunchKernelGGL(finalize_ahead_kernel, dim3(1), dim3(kBlock), 0, s, partials, n, 1.0 / double(N), ahead, ahead64, avg,
+    hipLaunchKernelGGL(finalize_ahead_kernel, dim3(1), dim3(kFinalBlock), 0, s, partials, n, 1.0 / double(N), ahead, ahead64, avg,
                        avg64);
     return hipGetLastError();
 }

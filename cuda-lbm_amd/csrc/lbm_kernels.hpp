@@ -60,6 +60,16 @@ hipError_t launch_march(int coll, int storage, const StepParams& p, const MarchP
 hipError_t launch_march_f32(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s);
 hipError_t launch_march_f16(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s);
 hipError_t launch_march_bf16(int coll, int steps, const StepParams& p, const MarchGrid& m, bool edge, bool wide, hipStream_t s);
+// The look-ahead step of CM<OptimalAdapter> (launch_step_ahead) in marching strips of one
+// wavefront: as there, with one partial triple per strip (march_strips of them). steps 0: not
+// for this grid.
+MarchPolicy march_ahead_policy(int nx, int ny, long long plane, int storage, bool edge);
+long long march_strips(const StepParams& p, const MarchPolicy& lp);
+hipError_t launch_march_ahead(int storage, const StepParams& p, const MarchPolicy& lp, const uint8_t* row_info, double* partials,
+                              hipStream_t s);
+hipError_t launch_march_ahead_f32(const StepParams& p, const MarchGrid& m, bool edge, bool wide, double* partials, hipStream_t s);
+hipError_t launch_march_ahead_f16(const StepParams& p, const MarchGrid& m, bool edge, bool wide, double* partials, hipStream_t s);
+hipError_t launch_march_ahead_bf16(const StepParams& p, const MarchGrid& m, bool edge, bool wide, double* partials, hipStream_t s);
 // to_store = 1: edge nodes of `buf` -> store; 0: store -> edge nodes of `buf`.
 hipError_t launch_edge_copy(int storage, void* buf, void* store, long long plane, int nx, int ny, int px, int py,
                             int to_store, hipStream_t s);

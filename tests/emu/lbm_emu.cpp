@@ -287,7 +287,7 @@ int run_t(const lbm_config& c, const uint8_t* flags, const float* rho, const flo
             local = local && !flag_reads_neighbour(fl[n]);
     const bool two = two_ty != 0 && !adapt && !(c.quirks & LBM_QUIRK_STALE_REST) && local;
     // CM<OptimalAdapter> with same-step averages: look-ahead launches where the library uses them
-    const bool ahead = two_ty < 0 && adapt && c.adapter_mode == LBM_ADAPTER_SAME_STEP &&
+    const bool ahead = (two_ty < 0 || two_ty / 1000000 == 2) && adapt && c.adapter_mode == LBM_ADAPTER_SAME_STEP &&
                        !(c.quirks & LBM_QUIRK_STALE_REST) && local;
     bool ahead_valid = false, ahead_edges = false;
     float ahead_avg[3] = {0.f, 0.f, 0.f};
@@ -350,7 +350,7 @@ int run_t(const lbm_config& c, const uint8_t* flags, const float* rho, const flo
             p.edge_next = n_edge ? edge[1 - edge_cur].data() : nullptr;
             p.n_edge = n_edge;
             p.edge_all = nsteps - s - per < 2;
-            if (march_s && per == march_s) {
+            if (march_s > 2 && per == march_s) {
                 if (march_s == 4) launch_march_emu<COLL, STORE, 4, 0>(p, march_w, march_h, reverse, nullptr);
                 else launch_march_emu<COLL, STORE, 6, 0>(p, march_w, march_h, reverse, nullptr);
             } else if (two_ty < 0) {  // marching strips: -(W * 1000 + H)
@@ -394,8 +394,8 @@ int run_t(const lbm_config& c, const uint8_t* flags, const float* rho, const flo
             p.edge_prev = n_edge ? edge[edge_cur].data() : nullptr;
             p.edge_next = n_edge ? edge[1 - edge_cur].data() : nullptr;
             p.n_edge = n_edge;
-            const int H = (-two_ty) % 1000;
-            launch_ahead_emu<COLL, STORE, 4>(p, H, reverse, partials);
+            if (march_s == 2) launch_march_emu<LBM_CM, STORE, 2, 1>(p, march_w, march_h, reverse, &partials);
+            else launch_ahead_emu<COLL, STORE, 4>(p, (-two_ty) % 1000, reverse, partials);
             // finalize: the averages used become the reported ones, the sums the next ones
             for (int k = 0; k < 3; k++) {
                 avg[k] = ahead_avg[k];
@@ -489,7 +489,7 @@ extern "C" int emu_run(const lbm_config* c, int seg, int two_ty, int reverse, co
         if ((W != 4 && W != 8) || H < 1) return -1;
     } else if (two_ty >= 1000000) {  // marching launches; narrower grids take the other forms
         const int S = two_ty / 1000000, W = (two_ty / 1000) % 1000, H = two_ty % 1000;
-        if ((S != 4 && S != 6) || W < 1 || W > kMarchLanes - 2 * (S - 1) || H < 1 || H + 2 * (S - 1) > kMarchMaxRows ||
+        if ((S != 2 && S != 4 && S != 6) || W < 1 || W > kMarchLanes - 2 * (S - 1) || H < 1 || H + 2 * (S - 1) > kMarchMaxRows ||
             c->nx < kMarchMinSide || c->ny < kMarchMinSide)
             return -1;
     } else if (two_ty != 0 && two_ty != 6 && two_ty != 14) {

@@ -68,6 +68,20 @@ def test_emulated_march_inner_flags():
         assert np.array_equal(f1, f2), form
 
 
+@pytest.mark.parametrize("form", [(2, 62, 8), (2, 62, 3), (2, 9, 48)], ids=lambda f: "w%dh%d" % f[1:])
+@pytest.mark.parametrize("storage", [A.LBM_F32, A.LBM_F16_SHIFTED], ids=["f32", "f16"])
+@pytest.mark.parametrize("layout", ["periodic", "channel", "cavity_mw", "zouhe_top", "open"])
+def test_emulated_march_lookahead_adapter(layout, storage, form):
+    # the look-ahead step in marching strips against the LDS strips: the same state bit for bit
+    # (4 steps: the rate of the adapter may flip a node at its threshold under another order of
+    # the means' sums after more), the same means up to the order of their FP64 sums
+    case = layout_case(layout, 150, 37, A.LBM_CM, adapter=A.LBM_OPTIMAL_ADAPTER, storage=storage)
+    f1, r1, u1, a1 = run_emu(case, 4, two_ty=(4, 8))
+    f2, r2, u2, a2 = run_emu(case, 4, two_ty=_code(form), reverse=True)
+    assert np.max(np.abs(a1 - a2) / np.abs(a1)) <= 1e-12
+    assert np.array_equal(r1, r2) and np.array_equal(u1, u2) and np.array_equal(f1, f2)
+
+
 # grids that take each marching form of the library: four and six steps, with and without edges,
 # narrow and wide workgroups; 13 steps also run a remainder
 GPU_GRIDS = [("periodic", 1030, 900), ("cavity_mw", 1030, 900), ("channel", 1016, 911), ("zouhe_top", 1001, 910),
