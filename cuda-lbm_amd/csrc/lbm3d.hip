@@ -71,13 +71,22 @@ __global__ __launch_bounds__(256) void step3_pre_kernel(Step3Params p, const int
     step3_node<COLL, STORE, BUF, GUO>(p, x, y, z);
 }
 
-// init_kernel<3> + init_node (init.cuh:10-43): both buffers = f_eq(rho, u), u AoS [N][3].
+// init_kernel<3> + init_node (init.cuh:10-43): f = f_back = f_eq(rho, u), u AoS [N][3]. Bound by
+// its writes; of f_back only the slots a step may read are written (nodes on a non-periodic face,
+// or all under the stale-rest quirk: `both`), the first step overwrites the rest.
 template <int STORE>
 __global__ void init3_kernel(void* a, void* b, long long plane, long long N, float rho0, float lin_ec,
-                             const float* rho, const float* u) {
+                             const float* rho, const float* u, int nx, int ny, int nz, int px, int py, int pz, int both) {
     const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= N) return;
     using T = typename Store3<STORE>::T;
+    bool back = both != 0;
+    if (!back && !(px && py && pz)) {
+        const uint32_t row = uint32_t(n) / uint32_t(nx), x = uint32_t(n) - row * uint32_t(nx);  // N < 2^31
+        const uint32_t z = row / uint32_t(ny), y = row - z * uint32_t(ny);
+        back = (!px && (x == 0 || x == uint32_t(nx - 1))) || (!py && (y == 0 || y == uint32_t(ny - 1))) ||
+               (!pz && (z == 0 || z == uint32_t(nz - 1)));
+    }
     float g[Q];
     for (int q = 0; q < Q; q++) g[q] = 0.0f;
     // f_eq is the BGK update at omega = 1 of any state with these moments and no force
@@ -86,7 +95,7 @@ __global__ void init3_kernel(void* a, void* b, long long plane, long long N, flo
     for (int q = 0; q < Q; q++) {
         const T v = Store3<STORE>::enc(g[q], q, rho0);
         static_cast<T*>(a)[q * plane + n] = v;
-        static_cast<T*>(b)[q * plane + n] = v;
+        if (back) static_cast<T*>(b)[q * plane + n] = v;
     }
 }
 
@@ -799,15 +808,17 @@ int lbm3d_init_from_macros(lbm3d_ctx* ctx, const float* rho, const float* u, int
         du = t + ctx->N;
     }
     const dim3 g(grid1(ctx->N)), b(256);
+    const int px = ctx->cfg.periodic_x != 0, py = ctx->cfg.periodic_y != 0, pz = ctx->cfg.periodic_z != 0;
+    const int both = (ctx->cfg.quirks & LBM_QUIRK_STALE_REST) ? 1 : 0;
     switch (ctx->cfg.storage) {
         case LBM_F32:
-            hipLaunchKernelGGL(init3_kernel<LBM_F32>, g, b, 0, ctx->stream, ctx->buf[0], ctx->buf[1], ctx->plane, ctx->N, ctx->cfg.rho0, ctx->lin_ec(), dr, du);
+            hipLaunchKernelGGL(init3_kernel<LBM_F32>, g, b, 0, ctx->stream, ctx->buf[0], ctx->buf[1], ctx->plane, ctx->N, ctx->cfg.rho0, ctx->lin_ec(), dr, du, ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz, px, py, pz, both);
             break;
         case LBM_F16_SHIFTED:
-            hipLaunchKernelGGL(init3_kernel<LBM_F16_SHIFTED>, g, b, 0, ctx->stream, ctx->buf[0], ctx->buf[1], ctx->plane, ctx->N, ctx->cfg.rho0, ctx->lin_ec(), dr, du);
+            hipLaunchKernelGGL(init3_kernel<LBM_F16_SHIFTED>, g, b, 0, ctx->stream, ctx->buf[0], ctx->buf[1], ctx->plane, ctx->N, ctx->cfg.rho0, ctx->lin_ec(), dr, du, ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz, px, py, pz, both);
             break;
         default:
-            hipLaunchKernelGGL(init3_kernel<LBM_BF16_SHIFTED>, g, b, 0, ctx->stream, ctx->buf[0], ctx->buf[1], ctx->plane, ctx->N, ctx->cfg.rho0, ctx->lin_ec(), dr, du);
+            hipLaunchKernelGGL(init3_kernel<LBM_BF16_SHIFTED>, g, b, 0, ctx->stream, ctx->buf[0], ctx->buf[1], ctx->plane, ctx->N, ctx->cfg.rho0, ctx->lin_ec(), dr, du, ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.nz, px, py, pz, both);
             break;
     }
     hipError_t e = hipGetLastError();

@@ -625,13 +625,11 @@ int lbm_init_from_macros(lbm_ctx* ctx, const float* rho, const float* u, int on_
         drho = t;
         du = t + ctx->N;
     }
-    InitParams ip{drho, du, ctx->buf[0], ctx->buf[1], ctx->plane, (long long)ctx->N, ctx->cfg.rho0};
+    InitParams ip{drho, du, ctx->buf[0], ctx->buf[1], ctx->plane, (long long)ctx->N, ctx->cfg.rho0,
+                  ctx->d_rho, ctx->d_ux, ctx->d_uy, ctx->cfg.nx, ctx->cfg.ny, ctx->cfg.periodic_x, ctx->cfg.periodic_y,
+                  (ctx->cfg.quirks & LBM_QUIRK_STALE_REST) ? 1 : 0};
     hipError_t e = launch_init(ctx->cfg.storage, ip, ctx->stream);
     if (e != hipSuccess) return ctx->hip_fail(e, "init launch");
-    e = hipMemcpyAsync(ctx->d_rho, drho, ctx->N * 4, hipMemcpyDeviceToDevice, ctx->stream);
-    if (e != hipSuccess) return ctx->hip_fail(e, "rho copy");
-    e = launch_aos_to_soa(du, (long long)ctx->N, ctx->d_ux, ctx->d_uy, ctx->stream);
-    if (e != hipSuccess) return ctx->hip_fail(e, "u split");
     if (!on_device) {
         e = hipStreamSynchronize(ctx->stream);
         if (e != hipSuccess) return ctx->hip_fail(e, "hipStreamSynchronize");
@@ -723,13 +721,12 @@ int lbm_get_macros(lbm_ctx* ctx, float* rho, float* u, int on_device) {
     if (rc) return rc;
     hipError_t e;
     if (on_device) {
-        if (rho) {
+        if (u) {
+            e = launch_macros_to_aos(ctx->d_ux, ctx->d_uy, (long long)ctx->N, u, rho ? ctx->d_rho : nullptr, rho, ctx->stream);
+            if (e != hipSuccess) return ctx->hip_fail(e, "u interleave");
+        } else if (rho) {
             e = hipMemcpyAsync(rho, ctx->d_rho, ctx->N * 4, hipMemcpyDeviceToDevice, ctx->stream);
             if (e != hipSuccess) return ctx->hip_fail(e, "rho copy");
-        }
-        if (u) {
-            e = launch_macros_to_aos(ctx->d_ux, ctx->d_uy, (long long)ctx->N, u, ctx->stream);
-            if (e != hipSuccess) return ctx->hip_fail(e, "u interleave");
         }
         return LBM_OK;
     }
@@ -740,7 +737,7 @@ int lbm_get_macros(lbm_ctx* ctx, float* rho, float* u, int on_device) {
     if (u) {
         rc = ctx->scratch(ctx->N * 8);
         if (rc) return rc;
-        e = launch_macros_to_aos(ctx->d_ux, ctx->d_uy, (long long)ctx->N, static_cast<float*>(ctx->tmp), ctx->stream);
+        e = launch_macros_to_aos(ctx->d_ux, ctx->d_uy, (long long)ctx->N, static_cast<float*>(ctx->tmp), nullptr, nullptr, ctx->stream);
         if (e != hipSuccess) return ctx->hip_fail(e, "u interleave");
         e = hipMemcpyAsync(u, ctx->tmp, ctx->N * 8, hipMemcpyDeviceToHost, ctx->stream);
         if (e != hipSuccess) return ctx->hip_fail(e, "u copy");

@@ -17,6 +17,9 @@ struct InitParams {
     void* buf1;
     long long plane, N;
     float rho0;
+    float *out_rho, *out_ux, *out_uy;  // the fields, as a step stores them
+    int nx, ny, px, py;
+    int both;                          // every slot of buf1 too (LBM_QUIRK_STALE_REST reads them)
 };
 
 // Launch shape of the fused step: workgroup size, XCD-contiguous workgroup order,
@@ -87,8 +90,8 @@ hipError_t launch_finalize_ahead(const double* partials, long long n, long long 
 hipError_t launch_init(int storage, const InitParams& p, hipStream_t s);
 hipError_t launch_pops_to_f32(int storage, const void* buf, long long plane, long long N, float rho0, float* out, hipStream_t s);
 hipError_t launch_pops_from_f32(int storage, void* b0, void* b1, long long plane, long long N, float rho0, const float* in, hipStream_t s);
-hipError_t launch_macros_to_aos(const float* ux, const float* uy, long long N, float* u, hipStream_t s);
-hipError_t launch_aos_to_soa(const float* u, long long N, float* ux, float* uy, hipStream_t s);
+// u AoS, and with rho_in also a copy of the density.
+hipError_t launch_macros_to_aos(const float* ux, const float* uy, long long N, float* u, const float* rho_in, float* rho_out, hipStream_t s);
 long long reduce_partials_needed(long long N);
 hipError_t launch_reduce(int kind, const float* rho, const float* ux, const float* uy, const float* ref, long long N,
                          double* partials, double* out3, hipStream_t s);
