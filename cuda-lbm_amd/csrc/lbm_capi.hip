@@ -190,7 +190,7 @@ int lbm_ctx::ahead_step(bool write_macros) {
     p.edge_next = d_edge[1 - edge_cur];
     p.n_edge = n_edge;
     MarchPolicy mp;
-    if (flags_march) mp = march_ahead_policy(cfg.nx, cfg.ny, plane, cfg.storage, d_flags || n_edge > 0);
+    if (flags_march) mp = march_ahead_policy(cfg.nx, cfg.ny, plane, cfg.storage, d_flags || n_edge > 0, cfg.periodic_x != 0);
     const Step2Policy lp = ahead_policy(plane, cfg.storage);
     const long long np = mp.steps ? march_strips(p, mp) : ahead_partials_needed(p, lp);
     rc = ensure_partials(np);
@@ -238,7 +238,7 @@ int lbm_ctx::multi_step(int steps_left, bool last, int* done) {
         if (e != hipSuccess) return hip_fail(e, "edge save launch");
     }
     MarchPolicy mp;
-    if (flags_march) mp = march_policy(cfg.nx, cfg.ny, plane, cfg.storage, cfg.collision, d_flags || n_edge > 0, steps_left);
+    if (flags_march) mp = march_policy(cfg.nx, cfg.ny, plane, cfg.storage, cfg.collision, d_flags || n_edge > 0, cfg.periodic_x != 0, steps_left);
     const int n = mp.steps ? mp.steps : 2;
     const bool write_macros = last && n == steps_left;
     StepParams p = step_params(cur, write_macros);

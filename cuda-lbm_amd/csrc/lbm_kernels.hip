@@ -2,6 +2,7 @@
 #include "lbm_kernels.hpp"
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cmath>
 
 namespace lbm {
@@ -581,17 +582,22 @@ Step2Policy step2_policy(long long plane, int storage, int coll) {
 
 // Rows per marching strip. The height balances the halo rows (S - 1 + h per h) against the
 // number of wavefronts: the cost is wavefronts per SIMD, rounded up, times rows, with a penalty
-// for one or two wavefronts per SIMD, which leave the vector ALU idle while they wait.
-static int march_height(int nx, int ny, int w, int steps, bool edge) {
+// for one or two wavefronts per SIMD, which leave the vector ALU idle while they wait. With walls
+// at x = 0 and NX-1 every row of the strips there is special and those strips end last: half a
+// wavefront's rows more, which prefers shorter strips, and they hide a last round of 1 %. Cavity
+// 1024^2 MRT F32, us per step at h 5/6/7/9/10: 9.2/8.7/9.3/8.8/9.3; 1100x900 BGK at h 6/7/9:
+// 7.9/7.8/8.1; 1500^2 at h 10/13/20: 14.0/13.7/15.5. Without such walls 4096x1024 takes 25.6 at
+// h 36, 0.5 % over two rounds, against 21.2 at h 24.
+static int march_height(int nx, int ny, int w, int steps, bool edge, bool side) {
     const long long sx = (nx + w - 1) / w;
     const int resident = edge ? 4 : 5;  // wavefronts per SIMD
     double best = 1e30;
     int height = 1;
     for (int h = 1; h <= 48; h++) {
         const double n = double(sx * ((ny + h - 1) / h)) / double(kSimds), rows = h + steps - 1;
-        const double c = std::ceil(n);
+        const double c = std::max(1.0, std::ceil(n - (side ? 0.01 : 0.0)));
         const double idle = c <= 1 ? 1.7 : (c <= 2 ? 1.1 : (c <= 3 ? 1.03 : 1.0));
-        const double cost = (c <= resident ? c * idle : n + 0.5) * rows;
+        const double cost = ((c <= resident ? c * idle : n + 0.5) + (side ? 0.5 : 0.0)) * rows;
         if (cost < best) {
             best = cost;
             height = h;
@@ -608,17 +614,17 @@ static int march_height(int nx, int ny, int w, int steps, bool edge) {
 //   periodic 8192^2 F32: BGK 505 -> 223 (6x48x32 wide; 6x54x32 259, 4x48x32 312),
 //                        MRT 511 -> 256..262 (6x48x48, 6x54x32), CM 530 -> 308 (6x54x32; 4x48x32 336)
 //   periodic 8192^2 F16: BGK 336 -> 215..220 (4x58), MRT 361 -> 245
-//   channel   4096x1024 CM BF16 36.7 -> 28 (4x58), MRT F32 41.8 -> 24 (4x58x24; 6x54x16 25.5)
-//   cavity    1024^2 MRT F32 11.1 -> 9.3 (4x58x10)     4000x3000 BGK F32 107 -> 49 (6x54x32; 4x58x32 64)
-//   cavity    2048^2 MRT F16 36.0 -> 25.3, F32 45.1 -> 24.1 (4x58)
-//   walls on small grids: cavity 512^2 5.08 -> 5.14, 256^2 CM 3.55 -> 4.31, 6000x60 5.50 -> 5.93,
-//   channel 700^2 CM 6.43 -> 7.31, cavity 777x611 MRT F16 6.6 -> 7.0: there the strips along the
+//   channel   4096x1024 CM BF16 34.8 -> 24.4 (4x58x24), MRT F32 40.7 -> 21.2 (4x58x24)
+//   cavity    1024^2 MRT F32 11.2 -> 8.7 (4x58x6)     4000x3000 BGK F32 107 -> 49 (6x54x32; 4x58x32 50)
+//   cavity    2048^2 MRT F16 36.0 -> 25.3, F32 44.4 -> 25.1 (4x58x12)
+//   walls on small grids: cavity 512^2 4.93 -> 5.00, 256^2 CM 3.48 -> 4.23, 6000x60 5.50 -> 5.93,
+//   channel 700^2 CM 6.19 -> 6.59, cavity 777x611 MRT F16 6.54 -> 7.23: there the strips along the
 //   walls are a large share and set the launch time, so up to 48 MB walled grids keep the tiles.
 // Six steps pay once the populations leave the Infinity Cache (the launch is then bound by HBM
 // at four steps, by the vector ALU at six), later for CM (more arithmetic) and walled grids.
 // Aligned 48-column strips, four to a workgroup, write whole 64-byte granules and keep the
 // neighbours' shared lines in L2; the 14 % of lanes they idle only pay in HBM and for BGK.
-MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll, bool edge, int steps_left) {
+MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll, bool edge, bool px, int steps_left) {
     MarchPolicy lp;
     const bool f32 = storage == LBM_F32;
     if (nx < kMarchMinSide || ny < kMarchMinSide || steps_left < 4) return lp;
@@ -637,7 +643,7 @@ MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll,
         }
         return lp;
     }
-    lp.h = march_height(nx, ny, lp.w, lp.steps, edge);
+    lp.h = march_height(nx, ny, lp.w, lp.steps, edge, !px);
     return lp;
 }
 
@@ -660,7 +666,7 @@ hipError_t launch_march(int coll, int storage, const StepParams& p, const MarchP
 // F32 97.7 -> 85.2 (h 20..24; 16 104), F16 78.4 -> 65.7; 1024^2 F32 32.4 -> 27.2; 300x200 22.4
 // -> 12.3; 700x500 BF16 56 -> 17.9 (few strips: the LDS form marched 32 rows in each); beyond
 // the cache 6000x3000 F32 359 -> 339 at h 16 (359 at 32).
-MarchPolicy march_ahead_policy(int nx, int ny, long long plane, int storage, bool edge) {
+MarchPolicy march_ahead_policy(int nx, int ny, long long plane, int storage, bool edge, bool px) {
     MarchPolicy lp;
     const bool f32 = storage == LBM_F32;
     if (nx < kMarchMinSide || ny < kMarchMinSide) return lp;
@@ -668,7 +674,7 @@ MarchPolicy march_ahead_policy(int nx, int ny, long long plane, int storage, boo
     const double bytes = 2.0 * 9.0 * double(plane) * (f32 ? 4.0 : 2.0);
     lp.steps = 2;
     lp.w = kMarchLanes - 2;
-    lp.h = bytes > 600.0e6 ? 16 : march_height(nx, ny, lp.w, 2, edge);
+    lp.h = bytes > 600.0e6 ? 16 : march_height(nx, ny, lp.w, 2, edge, !px);
     return lp;
 }
 

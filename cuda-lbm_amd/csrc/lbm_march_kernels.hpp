@@ -38,17 +38,8 @@ template <int COLL, int STORE, int S, bool EDGE, int FORCED, int MODE>
 __device__ __forceinline__ void march_run(MarchLane<COLL, STORE, S, EDGE, FORCED, MODE>& w, const StepParams& p,
                                           const MarchGrid& m, MarchHist<S>* h, int l, MomAcc& acc) {
     const int n = w.iterations();
-    if (EDGE) {
-        const auto f = w.look(p, m, l);
-        w.rows = MarchRows{__builtin_amdgcn_ballot_w64(f.special), __builtin_amdgcn_ballot_w64(f.straight),
-                           __builtin_amdgcn_ballot_w64(f.moving), __builtin_amdgcn_ballot_w64(f.flag)};
-    }
     w.prefetch(p, 0);
     for (int i = 0; i < n; i++) {
-        if (EDGE) {  // opaque per iteration: no second copy of the march for strips without an x edge
-            w.xany = __builtin_amdgcn_readfirstlane(w.xany);
-            asm volatile("" : "+s"(w.xany));
-        }
         w.advance();
         if (i + 1 < n) w.prefetch(p, i + 1);
         __builtin_amdgcn_sched_barrier(0);  // the next row's loads are issued before this row's work
@@ -57,7 +48,9 @@ __device__ __forceinline__ void march_run(MarchLane<COLL, STORE, S, EDGE, FORCED
 }
 
 // WGW wavefronts per workgroup: neighbours along x, so that they start together and the cache
-// lines their strips share are in one L2 at one time. No wavefront waits for another.
+// lines their strips share are in one L2 at one time. No wavefront waits for another. On grids
+// with edges or flags a strip without any special row runs the plain body: the edge body's
+// branches over its rare code cost a wavefront 40 % even where none is taken.
 template <int COLL, int STORE, int S, bool EDGE, int FORCED, int MODE, int WGW>
 __global__ __launch_bounds__(kMarchLanes * WGW) void march_kernel(StepParams p, MarchGrid m, int nb, double* partials) {
     __shared__ MarchHist<S> hist[EDGE && S > 2 ? WGW : 1];
@@ -67,10 +60,24 @@ __global__ __launch_bounds__(kMarchLanes * WGW) void march_kernel(StepParams p, 
     const int strip = lb * WGW + wv;
     if (strip >= m.n_strips) return;
     const int l = int(threadIdx.x % kMarchLanes);
+    MarchHist<S>* h = &hist[EDGE && S > 2 ? wv : 0];
     MomAcc acc{0.0, 0.0, 0.0};
     MarchLane<COLL, STORE, S, EDGE, FORCED, MODE> w;
     w.init(p, m, strip, l);
-    march_run(w, p, m, &hist[EDGE && S > 2 ? wv : 0], l, acc);
+    bool plain = false;
+    if (EDGE) {
+        const auto f = w.look(p, m, l);
+        w.rows = MarchRows{__builtin_amdgcn_ballot_w64(f.special), __builtin_amdgcn_ballot_w64(f.straight),
+                           __builtin_amdgcn_ballot_w64(f.moving), __builtin_amdgcn_ballot_w64(f.flag)};
+        plain = w.rows.special == 0;
+    }
+    if (plain) {
+        MarchLane<COLL, STORE, S, false, FORCED, MODE> v;
+        v.init(p, m, strip, l);
+        march_run(v, p, m, h, l, acc);
+    } else {
+        march_run(w, p, m, h, l, acc);
+    }
     if constexpr (MODE == 1) {
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
