@@ -462,11 +462,13 @@ int lbm3d_ctx::one_step(bool write_macros) {
     // once the two buffers do not fit the 256 MiB Infinity Cache (256^3 F16 382 -> 369, F32 +2 %);
     // on resident grids they push every write to HBM (us per step without / with: 100^3 CM F32,
     // 216 MB, 34 / 43; 128^3 F16, 226 MB, 40 / 50; duct 250x128x96 F16, 332 MB, 75 / 75; 64^3 F32
-    // 11 / 13). Stores that do not start on a line write it in parts, which costs more than the
-    // cached lines gain (tunnel 250x128x96 F32 206 / 230): then only flat launches use them.
+    // 11 / 13). Stores whose rows are not whole 64-byte write granules write parts of them, which
+    // costs more than the cached lines gain (tunnel 250x128x96 F32 209 / 234, 104x200x200 286 /
+    // 320, 250x200x200 F16 386 / 483; whole granules: 112x197x213 F32 286 / 258, 80x200x200
+    // 213 / 193, 224x200x200 F16 361 / 358): then only flat launches use them.
     constexpr double kNtBufferBytes = 268.0e6;
-    const bool lines = p.flat || (long long)cfg.nx * (long long)elem_bytes(cfg.storage) % 128 == 0;
-    p.nt = lines && 2.0 * Q * double(plane) * double(elem_bytes(cfg.storage)) > kNtBufferBytes ? 1 : 0;
+    const bool granules = p.flat || (long long)cfg.nx * (long long)elem_bytes(cfg.storage) % 64 == 0;
+    p.nt = granules && 2.0 * Q * double(plane) * double(elem_bytes(cfg.storage)) > kNtBufferBytes ? 1 : 0;
     if (p.flat) {
         magic_div(uint32_t(cfg.nx), p.div_x, p.shift_x);
         magic_div(uint32_t(cfg.ny), p.div_y, p.shift_y);
