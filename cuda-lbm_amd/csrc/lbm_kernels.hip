@@ -644,6 +644,12 @@ MarchPolicy march_policy(int nx, int ny, long long plane, int storage, int coll,
         return lp;
     }
     lp.h = march_height(nx, ny, lp.w, lp.steps, edge, !px);
+    // 16-bit storage converts and rounds at every stage, all of it in one wavefront's chain. Once
+    // strips are taller than a row and before they fill the SIMDs, the chain of MRT and CM is
+    // longer than two tile launches (periodic, BF16, tiles -> 4x58): CM 117x373 2.74 -> 3.20,
+    // 300x400 3.23 -> 3.85, 512^2 4.68 -> 4.91, 700x600 5.89 -> 5.67, MRT 117x373 2.57 -> 2.89,
+    // 300x400 3.46 -> 3.43; at one row (128^2) CM 2.89 -> 2.66.
+    if (!f32 && lp.h > 1 && ((coll == LBM_CM && bytes <= 14.0e6) || (coll == LBM_MRT && bytes <= 4.0e6))) return MarchPolicy{};
     return lp;
 }
 
