@@ -539,11 +539,18 @@ int lbm_set_flags(lbm_ctx* ctx, const uint8_t* flags, int on_device) {
     std::vector<uint8_t> rowc(size_t(ny) * 2, 0);  // row classes, then march_row_info()
     bool any = false, local = true, march = true;
     for (int y = 0; y < ny; y++) {
+        const uint8_t* row = h.data() + size_t(y) * nx;
         for (int x = 0; x < nx; x++) {
-            uint8_t f = h[size_t(y) * nx + x];
+            static_assert(LBM_FLUID == 0, "eight FLUID nodes are a zero word");
+            for (uint64_t eight; x + 8 <= nx; x += 8) {  // runs of FLUID nodes, the bulk of a grid
+                std::memcpy(&eight, row + x, 8);
+                if (eight) break;
+            }
+            if (x == nx) break;
+            const uint8_t f = row[x];
+            if (f == LBM_FLUID) continue;
             if (!flag_supported(f))
                 return ctx->fail(LBM_E_UNSUPPORTED, "BC flag %d at node (%d,%d) is not supported", int(f), x, y);
-            if (f == LBM_FLUID) continue;
             any = true;
             if (flag_reads_neighbour(f)) local = false;
             if (!march_flag(f)) march = false;
