@@ -60,17 +60,32 @@ def time_steps(solver, steps, warmup, torch, batches=BATCHES):
     return sorted(secs)[len(secs) // 2], secs
 
 
+def launch_steps(cfg, spl):
+    """Time steps of a full launch of a case whose `steps_per_launch` is spl (1, or 2 for
+    several): the library's rule for grids without flags that need the two-step forms."""
+    from lbm_amd import _abi as A
+
+    if spl == 1 or min(cfg.nx, cfg.ny) < 16:
+        return spl
+    f32 = cfg.storage == A.LBM_F32
+    walled = not (cfg.periodic_x and cfg.periodic_y)
+    nbytes = bytes_per_node(cfg.storage) * cfg.N
+    if (walled and nbytes <= 48e6) or nbytes // 2 >= 1 << 32:
+        return 2
+    return 6 if f32 and nbytes > (600e6 if walled or cfg.collision == A.LBM_CM else 256e6) else 4
+
+
 def run_case(case, steps, warmup, torch, batches=BATCHES):
     """MLUPS (median of `batches` batches of `steps` steps), and the bandwidth of the step
-    kernel: a launch advances `steps_per_launch` steps and moves every population once in and
+    kernel: a launch advances `launch_steps` steps and moves every population once in and
     once out (2*Q*s bytes per node), so the algorithmic bytes per node update are
-    2*Q*s / steps_per_launch."""
+    2*Q*s / launch_steps, reported as steps_per_launch."""
     from lbm_amd import Solver
 
     s = Solver(case.config)
     case.apply(s)
     secs, all_secs = time_steps(s, steps, warmup, torch, batches)
-    spl = s.steps_per_launch
+    spl = launch_steps(case.config, s.steps_per_launch)
     N = case.config.N
     mlups = N * steps / secs / 1e6
     B = bytes_per_node(case.config.storage)
@@ -115,7 +130,7 @@ def run_adjoint(torch, steps=2000, every=100):
 
     s.step(50)  # warm-up
     t_plain = timed(lambda: s.step(steps))
-    spl_plain = s.steps_per_launch
+    spl_plain = launch_steps(case.config, s.steps_per_launch)
     # the same forward with one step per launch: the kernel the backward's recompute runs
     one = sc.inverse_problem(512, steps=steps)
     one.config.steps_per_launch = 1
@@ -148,7 +163,7 @@ def run_adjoint(torch, steps=2000, every=100):
             "adjoint_vs_one_step_forward_cost": round(t_bwd / t_one, 3),
             "backward_includes": "segment recompute (1 forward step per adjoint step, two per launch with the "
                                  "intermediate state stored) + adjoint step; cost ratio against the default forward "
-                                 "(two steps per launch)",
+                                 "(several steps per launch)",
             "gradient_finite": ok}
 
 
@@ -243,7 +258,7 @@ def run_poiseuille(torch, steps=400, warmup=20, adapter_steps=100):
     """The force-driven Poiseuille channel (4096x1024 CM, periodic x, bounce-back walls,
     nu = 0.05, Guo force for u_max = 0.05), from rest.
 
-    - CM<NoAdapter>: MLUPS per storage (two steps per launch) and the 16-bit storages'
+    - CM<NoAdapter>: MLUPS per storage (four steps per launch) and the 16-bit storages'
       velocity against FP32 after the same steps.
     - CM<OptimalAdapter>, the configuration as specified: MLUPS per storage over its first
       warmup + adapter_steps steps. Each step is a moments pass, an FP64 finalize of the
@@ -680,10 +695,8 @@ def main():
                    "nodes": case.config.N, "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": head["GB_s"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": head["frac_hbm_peak"],
-                     "traffic": profiled_traffic("fused_step2_ldc1024_mrt_f32" if head["steps_per_launch"] == 2
-                                                 else "fused_step_ldc1024_mrt_f32"),
-                     "kernel": ("fused_step2_kernel<MRT,F32>" if head["steps_per_launch"] == 2
-                                else "fused_step_kernel<MRT,F32>"),
+                     "traffic": profiled_traffic("march_ldc1024_mrt_f32"),
+                     "kernel": "march_kernel<MRT,F32,4>",
                      "steps_per_launch": head["steps_per_launch"],
                      "kernel_avg_us": head["us_per_launch"],
                      "algorithmic_bytes_per_launch": head["bytes_per_node_per_launch"] * case.config.N,

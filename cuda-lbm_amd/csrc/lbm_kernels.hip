@@ -669,7 +669,7 @@ hipError_t launch_march(int coll, int storage, const StepParams& p, const MarchP
 }
 
 // Measured on MI355X, us per step with the finalize, against the LDS strips: channel 4096x1024
-// F32 97.7 -> 85.2 (h 20..24; 16 104), F16 78.4 -> 65.7; 1024^2 F32 32.4 -> 27.2; 300x200 22.4
+// F32 97.7 -> 81.2 (h 20..24; 16 104), F16 77.2 -> 57.0; 1024^2 F32 32.4 -> 27.2; 300x200 22.4
 // -> 12.3; 700x500 BF16 56 -> 17.9 (few strips: the LDS form marched 32 rows in each); beyond
 // the cache 6000x3000 F32 359 -> 339 at h 16 (359 at 32).
 MarchPolicy march_ahead_policy(int nx, int ny, long long plane, int storage, bool edge, bool px) {

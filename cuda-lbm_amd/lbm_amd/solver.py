@@ -41,7 +41,7 @@ class Config:
     wall_u: tuple = (0.0, 0.0)
     u_lid: float = 0.1
     quirks: int = 0
-    steps_per_launch: int = 0  # 0: two steps per launch where supported, 1: one
+    steps_per_launch: int = 0  # 0: several steps per launch where supported, 1: one
 
     def to_c(self) -> A.LbmConfig:
         c = A.LbmConfig()
@@ -157,7 +157,7 @@ class Solver:
 
     @property
     def steps_per_launch(self) -> int:
-        """Time steps per kernel launch lbm_step uses now (2 or 1)."""
+        """Time steps per kernel launch lbm_step uses now: 1, or 2 for several."""
         n = ctypes.c_int32()
         self._check(self.lib.lbm_get_steps_per_launch(self.h, ctypes.byref(n)))
         return n.value
