@@ -180,6 +180,14 @@ struct MarchEmu {
             rows.moving |= uint64_t(f.moving) << l;
             rows.flag |= uint64_t(f.flag) << l;
         }
+        if constexpr (EDGE) {
+            if (rows.special == 0) {  // the plain body, as in march_kernel
+                MarchEmu<COLL, STORE, S, false, FORCED, MODE> v(p, m);
+                v.run(strip);
+                acc = v.acc;
+                return;
+            }
+        }
         const int n = w[0].iterations();
         for (auto& x : w) {
             x.rows = rows;
